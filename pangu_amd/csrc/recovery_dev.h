@@ -213,6 +213,12 @@ __device__ inline double vsq_residual(const double U[9], const CenMetric &m, dou
 // scheme_1d_vsq.h:52-351 (K = previous primitive entropy).  The Newton
 // iteration starts from the v^2 of the previous primitives, as the
 // reference does, or from x0 when x0 >= 0 (the learned start).
+//
+// W, rho, p and u of an iterate are evaluated once, at the end of the step
+// that makes it, and serve the next step and the final reconstruction: the
+// same arguments give the same bits, and each evaluation is a pow, which
+// bounds this scheme (n + 1 of them for n steps; evaluating afresh at the top
+// of every step and after the last takes 2 n + 1).
 __device__ int c2p_1dvsq(const double U[9], double p[9], double gamma, const CenMetric &m,
                          int &iters, double x0 = -1.0) {
   iters = 0;
@@ -232,8 +238,8 @@ __device__ int c2p_1dvsq(const double U[9], double p[9], double gamma, const Cen
   double f = 1., df = 1., errx = 1., W = 0., pr, rho, uu;
   int i_extra = 0, doing_extra = 0, n_iter = 0;
   bool keep = true;
+  double Wf = w_of_vsq(D, K, x, gamma, pr, rho, uu);
   while (keep) {
-    double Wf = w_of_vsq(D, K, x, gamma, pr, rho, uu);
     {
       const double vsq = x;
       const double Wsq = Wf * Wf;
@@ -253,6 +259,7 @@ __device__ int c2p_1dvsq(const double U[9], double p[9], double gamma, const Cen
       x = fabs(x);
       const double Wo = W;
       W = w_of_vsq(D, K, x, gamma, pr, rho, uu);
+      Wf = W;
       errx = (W == 0.) ? fabs(W - Wo) : fabs((W - Wo) / W);
       errx += (x == 0.) ? fabs(x - xo) : fabs((x - xo) / x);
     }
@@ -272,11 +279,9 @@ __device__ int c2p_1dvsq(const double U[9], double p[9], double gamma, const Cen
   if (retval != 0) return retval * 100 + 1;
   const double vsq = x;
   if ((vsq >= 1.) || (vsq < 0.)) return 4;
-  double rho0;
-  W = w_of_vsq(D, K, vsq, gamma, pr, rho0, uu);
   const double Gamma = 1. / sqrt(1. - vsq);
-  if ((rho0 <= 0.) || (uu <= 0.)) return 5;
-  p[RHO] = rho0;
+  if ((rho <= 0.) || (uu <= 0.)) return 5;
+  p[RHO] = rho;
   p[ENY] = uu;
   noble_velocity(v, W, Gamma, p);
   return 0;
