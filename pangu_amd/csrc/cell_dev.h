@@ -31,20 +31,44 @@ __device__ __forceinline__ int64_t cen_index(const DevGeo &G, int k, int j, int 
   return ((int64_t)(G.has3d ? k : 0) * G.nj + j) * G.ni + i;
 }
 
+// gcov, g^{0m} and the lapse of a table entry, as far as form MF leaves them
+// open; the symmetric partner of a loaded entry shares its register.
+// comp(n) loads component n; GCON0 and ALPHA are the table's component
+// numbers of g^{00} and of 1/sqrt(-g^{00}).
+template <int MF, int GCON0, int ALPHA, class LD>
+__device__ __forceinline__ void load_metric(LD comp, double g[16], double gc0[4], double &alpha) {
+  if (MF == FORM_FLAT) {
+#pragma unroll
+    for (int n = 0; n < 16; ++n) g[n] = (n % 5) ? 0.0 : (n ? 1.0 : -1.0);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) gc0[n] = n ? 0.0 : -1.0;
+    alpha = 1.0;
+    return;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int slot = g_slot<MF>(r, c);
+      g[4 * r + c] = !g_open<MF>(r, c) ? 0.0 : (slot < 4 * r + c ? g[slot] : comp(slot));
+    }
+#pragma unroll
+  for (int n = 0; n < 4; ++n) gc0[n] = g0_open<MF>(n) ? comp(GCON0 + n) : 0.0;
+  alpha = comp(ALPHA);
+}
+
 // Loads of the centre table.
 struct CenLoad {
   double g[16], gc0[4], alpha, sg;
 };
+template <int MF = FORM_FULL>
 __device__ __forceinline__ void load_cen_state(const DevGeo &G, int64_t t, CenLoad &m) {
   const double *c = G.cen;
   const int64_t s = G.ncen;
   const uint32_t t32 = (uint32_t)t;
-#pragma unroll
-  for (int n = 0; n < 16; ++n) m.g[n] = ldc32(c, (CG_GCOV + n) * s, t32);
-#pragma unroll
-  for (int n = 0; n < 4; ++n) m.gc0[n] = ldc32(c, (CG_GCON + n) * s, t32);
-  m.alpha = ldc32(c, CG_ALPHA * s, t32);
-  m.sg = ldc32(c, CG_SG * s, t32);
+  auto comp = [&](int n) { return ldc32(c, n * s, t32); };
+  load_metric<MF, CG_GCON, CG_ALPHA>(comp, m.g, m.gc0, m.alpha);
+  m.sg = MF == FORM_FLAT ? 1.0 : comp(CG_SG);
 }
 
 }  // namespace pangu

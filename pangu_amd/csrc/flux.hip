@@ -20,7 +20,7 @@ namespace pangu {
 // One cell of k_fix_cons.  write = false computes without storing (a halo
 // cell of k_fix_flux_x1, which another workgroup owns); pout (optional)
 // receives the fixed primitives, every slot.
-template <bool FIX, bool CONS, bool HB, bool HK>
+template <int MF, bool FIX, bool CONS, bool HB, bool HK>
 __device__ __forceinline__ void fix_cons_cell(const KCtx &C, const KFields &F, uint8_t *const *mask, int b,
                                               int k, int j, int i, bool write, double *pout) {
   const DevBlock &B = C.blk[b];
@@ -40,7 +40,7 @@ __device__ __forceinline__ void fix_cons_cell(const KCtx &C, const KFields &F, u
 #pragma unroll
   for (int q = 0; q < NC; ++q) p[slot_of<HB, HK>(q)] = pp[q][id];
   CenLoad m;
-  load_cen_state(G, t, m);
+  load_cen_state<MF>(G, t, m);
   const Phys &P = C.ph;
   if (FIX) {
     const double small = 1.0e-20;
@@ -49,7 +49,7 @@ __device__ __forceinline__ void fix_cons_cell(const KCtx &C, const KFields &F, u
     double rho_floor = ldc32(G.cen, (int64_t)CG_RHOFL * G.ncen, (uint32_t)t);
     const double eng_floor = ldc32(G.cen, (int64_t)CG_ENGFL * G.ncen, (uint32_t)t);
     St st;
-    calc_state(p, m.g, m.gc0, m.alpha, st);
+    calc_state<MF, HB>(p, m.g, m.gc0, m.alpha, st);
     const double rho = p[RHO], ug = p[ENY];
     uint8_t mk = 0;
     if (rho_floor < ug / sms) rho_floor = ug / sms;
@@ -68,8 +68,9 @@ __device__ __forceinline__ void fix_cons_cell(const KCtx &C, const KFields &F, u
     }
     const double u1 = p[UX1], u2 = p[UX2], u3 = p[UX3];
     const double *g = m.g;
-    const double uvsq = g[5] * u1 * u1 + g[10] * u2 * u2 + g[15] * u3 * u3 +
-                        2.0 * (g[6] * u1 * u2 + g[7] * u1 * u3 + g[11] * u2 * u3);
+    double uvsq = g[5] * u1 * u1 + g[10] * u2 * u2 + g[15] * u3 * u3;
+    if (MF == FORM_FULL) uvsq = uvsq + 2.0 * (g[6] * u1 * u2 + g[7] * u1 * u3 + g[11] * u2 * u3);
+    if (MF == FORM_POLOIDAL) uvsq = uvsq + 2.0 * (g[7] * u1 * u3);
     const double umax2 = P.lorentz_max * P.lorentz_max - 1.0;
     if (umax2 > 0.0 && uvsq > umax2) {
       const double f = sqrt(umax2 / kmax(uvsq, small));
@@ -115,19 +116,19 @@ __device__ __forceinline__ void fix_cons_cell(const KCtx &C, const KFields &F, u
   }
   if (CONS && interior && write) {
     St st;
-    calc_state(p, m.g, m.gc0, m.alpha, st);
+    calc_state<MF, HB>(p, m.g, m.gc0, m.alpha, st);
     double f[NPRIM];
-    contravariant_flux<0>(P.gamma, p, st, m.sg, f);
+    contravariant_flux<0, HB>(P.gamma, p, st, m.sg, f);
 #pragma unroll
     for (int q = 0; q < NC; ++q) __builtin_nontemporal_store(f[slot_of<HB, HK>(q)], &glb(F.cons[b * NC + q])[id]);
   }
 }
 
-template <bool FIX, bool CONS, bool HB, bool HK>
+template <int MF, bool FIX, bool CONS, bool HB, bool HK>
 __global__ __launch_bounds__(256) void k_fix_cons(KCtx C, KFields F, uint8_t *const *mask, Range3 R) {
   int b, k, j, i;
   if (!decode_tile(C, R, b, k, j, i)) return;
-  fix_cons_cell<FIX, CONS, HB, HK>(C, F, mask, b, k, j, i, true, nullptr);
+  fix_cons_cell<MF, FIX, CONS, HB, HK>(C, F, mask, b, k, j, i, true, nullptr);
 }
 
 // ------------------------------------------------------------- flux sweep
@@ -139,7 +140,7 @@ __global__ __launch_bounds__(256) void k_fix_cons(KCtx C, KFields F, uint8_t *co
 // lower face of cell (k, j, i) along DIR: face metric, fluid states, fast
 // speeds, the four contravariant fluxes and the Riemann combine, from the
 // reconstructed left (pl) and right (pr) primitives.
-template <int DIR, int RS, bool HB, bool HK>
+template <int DIR, int RS, bool HB, bool HK, int MF = FORM_FULL>
 __device__ __forceinline__ void face_flux(const KCtx &C, const KFields &F, double *const *alfven, int b,
                                           int k, int j, int i, const double pl[NPRIM],
                                           const double pr[NPRIM]) {
@@ -147,37 +148,36 @@ __device__ __forceinline__ void face_flux(const KCtx &C, const KFields &F, doubl
   const int64_t id = ((int64_t)k * B.n[1] + j) * B.n[0] + i;
   constexpr int NC = ncomp<HB, HK>();
   const DevGeo &G = C.geo[B.geo];
-  double g[16], gc0[4], gdd, sg, alpha, valid;
-  if (DIR == 3 && !G.face[2]) {
+  double g[16], gc0[4], gdd = 1.0, sg = 1.0, alpha;
+  if (MF != FORM_FULL && DIR == 3) {  // no form but FULL depends on x3: the centre table serves
     const uint32_t t = (uint32_t)cen_index(G, k, j, i);
-    const double *c = G.cen;
-    const uint32_t s = (uint32_t)G.ncen;
-#pragma unroll
-    for (int n = 0; n < 16; ++n) g[n] = ldc32(c, (int64_t)(CG_GCOV + n) * s, t);
-#pragma unroll
-    for (int n = 0; n < 4; ++n) gc0[n] = ldc32(c, (int64_t)(CG_GCON + n) * s, t);
-    gdd = ldc32(c, (int64_t)(CG_GCON + 15) * s, t);
-    sg = ldc32(c, (int64_t)CG_SG * s, t);
-    alpha = ldc32(c, (int64_t)CG_ALPHA * s, t);
-    valid = 1.0;
+    auto comp = [&](int n) { return ldc32(G.cen, (int64_t)n * (uint32_t)G.ncen, t); };
+    load_metric<MF, CG_GCON, CG_ALPHA>(comp, g, gc0, alpha);
+    if (MF != FORM_FLAT) {
+      gdd = comp(CG_GCON + 15);
+      sg = comp(CG_SG);
+    }
+  } else if (DIR == 3 && !G.face[2]) {
+    const uint32_t t = (uint32_t)cen_index(G, k, j, i);
+    auto comp = [&](int n) { return ldc32(G.cen, (int64_t)n * (uint32_t)G.ncen, t); };
+    load_metric<MF, CG_GCON, CG_ALPHA>(comp, g, gc0, alpha);
+    gdd = comp(CG_GCON + 15);
+    sg = comp(CG_SG);
   } else {
     const int d = DIR - 1;
     const uint32_t t = (uint32_t)(((G.has3d ? k : 0) * G.fj[d] + j) * G.fi[d] + i);
-    const double *c = G.face[d];
-    const uint32_t s = (uint32_t)G.nface[d];
-#pragma unroll
-    for (int n = 0; n < 16; ++n) g[n] = ldc32(c, (int64_t)(FG_GCOV + n) * s, t);
-#pragma unroll
-    for (int n = 0; n < 4; ++n) gc0[n] = ldc32(c, (int64_t)(FG_GCON0 + n) * s, t);
-    gdd = ldc32(c, (int64_t)FG_GCONDD * s, t);
-    sg = ldc32(c, (int64_t)FG_SG * s, t);
-    alpha = ldc32(c, (int64_t)FG_ALPHA * s, t);
-    valid = ldc32(c, (int64_t)FG_VALID * s, t);
+    auto comp = [&](int n) { return ldc32(G.face[d], (int64_t)n * (uint32_t)G.nface[d], t); };
+    load_metric<MF, FG_GCON0, FG_ALPHA>(comp, g, gc0, alpha);
+    if (MF != FORM_FLAT) {
+      gdd = comp(FG_GCONDD);
+      sg = comp(FG_SG);
+    }
   }
   double *const al = alfven[b * 3 + (DIR - 1)];
   const uint32_t id32 = (uint32_t)id;
-  if (valid == 0.0) {
-    // singular face metric (polar axis): zero flux and wave speed
+  // a singular face metric (polar axis; its table entry holds alpha = 0)
+  // has zero flux and wave speed
+  if (MF != FORM_FLAT && alpha == 0.0) {
     st32(al, id32, 0.0);
 #pragma unroll
     for (int q = 0; q < NC; ++q) st32(F.flux[DIR - 1][b * NC + q], id32, 0.0);
@@ -185,20 +185,20 @@ __device__ __forceinline__ void face_flux(const KCtx &C, const KFields &F, doubl
   }
   const double gam = C.ph.gamma;
   St sl, sr;
-  calc_state(pl, g, gc0, alpha, sl);
-  calc_state(pr, g, gc0, alpha, sr);
+  calc_state<MF, HB>(pl, g, gc0, alpha, sl);
+  calc_state<MF, HB>(pr, g, gc0, alpha, sr);
   double vmaxL, vminL, vmaxR, vminR;
-  fast_ms<DIR>(gam, pl, sl, gc0[0], gc0[DIR], gdd, vmaxL, vminL);
-  fast_ms<DIR>(gam, pr, sr, gc0[0], gc0[DIR], gdd, vmaxR, vminR);
+  fast_ms<DIR, MF, HB>(gam, pl, sl, gc0[0], gc0[DIR], gdd, vmaxL, vminL);
+  fast_ms<DIR, MF, HB>(gam, pr, sr, gc0[0], gc0[DIR], gdd, vmaxR, vminR);
   const double cmax = fabs(kmax(kmax(0., vmaxL), vmaxR));
   const double cmin = fabs(kmax(kmax(0., -vminL), -vminR));
   const double cc = kmax(cmax, cmin);
   st32(al, id32, cc);
   double UL[NPRIM], UR[NPRIM], FL[NPRIM], FR[NPRIM];
-  contravariant_flux<0>(gam, pl, sl, sg, UL);
-  contravariant_flux<0>(gam, pr, sr, sg, UR);
-  contravariant_flux<DIR>(gam, pl, sl, sg, FL);
-  contravariant_flux<DIR>(gam, pr, sr, sg, FR);
+  contravariant_flux<0, HB>(gam, pl, sl, sg, UL);
+  contravariant_flux<0, HB>(gam, pr, sr, sg, UR);
+  contravariant_flux<DIR, HB>(gam, pl, sl, sg, FL);
+  contravariant_flux<DIR, HB>(gam, pr, sr, sg, FR);
   const double den = cmax + cmin + 1e-20, rden = 1.0 / den;
 #pragma unroll
   for (int q = 0; q < NC; ++q) {
@@ -213,7 +213,7 @@ __device__ __forceinline__ void face_flux(const KCtx &C, const KFields &F, doubl
 }
 
 
-template <int DIR, int LIM, int RS, bool HB, bool HK>
+template <int DIR, int LIM, int RS, bool HB, bool HK, int MF>
 __global__ __launch_bounds__(256) void k_flux(KCtx C, KFields F, double *const *alfven, Range3 R) {
   int b, k, j, i;
   if (!decode_tile(C, R, b, k, j, i)) return;
@@ -256,7 +256,7 @@ __global__ __launch_bounds__(256) void k_flux(KCtx C, KFields F, double *const *
       recon_mc(v[q][1], v[q][2], v[q][3], t1, pr[s]);
     }
   }
-  face_flux<DIR, RS, HB, HK>(C, F, alfven, b, k, j, i, pl, pr);
+  face_flux<DIR, RS, HB, HK, MF>(C, F, alfven, b, k, j, i, pl, pr);
 }
 
 // FixPrimitive + CalculateConservative (k_fix_cons) and the X1 sweep
@@ -320,7 +320,7 @@ __global__ __launch_bounds__(256) void k_fix_flux_x1(KCtx C, KFields F, uint8_t 
   double p[NPRIM];
 #pragma unroll
   for (int q = 0; q < NPRIM; ++q) p[q] = 0.0;
-  if (valid) fix_cons_cell<true, true, HB, HK>(C, F, mask, b, k, j, i, own, p);
+  if (valid) fix_cons_cell<FORM_FULL, true, true, HB, HK>(C, F, mask, b, k, j, i, own, p);
 #pragma unroll
   for (int q = 0; q < NPRIM; ++q) sp[q][x] = p[q];
   __syncthreads();
@@ -666,12 +666,19 @@ int launch_fix_cons(const LaunchCtx &L, const KFields &F, uint8_t *const *mask, 
   if (R.ntiles == 0) return 0;
   const dim3 g = tile_grid(R), wg(R.tile);
   const bool hb = L.k.iBX >= 0, hk = L.k.iKEL >= 0;
-#define FC(FX, CS, HB_, HK_) hipLaunchKernelGGL((k_fix_cons<FX, CS, HB_, HK_>), g, wg, 0, s, L.k, F, mask, R)
-#define FC2(FX, CS)                      \
-  if (hb && hk) FC(FX, CS, true, true);  \
-  else if (hb) FC(FX, CS, true, false);  \
-  else if (hk) FC(FX, CS, false, true);  \
-  else FC(FX, CS, false, false);
+  const int mf = metric_form(L.metric);
+#define FC(FX, CS, HB_, HK_)                                                                          \
+  if (mf == FORM_POLOIDAL)                                                                            \
+    hipLaunchKernelGGL((k_fix_cons<FORM_POLOIDAL, FX, CS, HB_, HK_>), g, wg, 0, s, L.k, F, mask, R);  \
+  else if (mf == FORM_FLAT)                                                                           \
+    hipLaunchKernelGGL((k_fix_cons<FORM_FLAT, FX, CS, HB_, HK_>), g, wg, 0, s, L.k, F, mask, R);      \
+  else                                                                                                \
+    hipLaunchKernelGGL((k_fix_cons<FORM_FULL, FX, CS, HB_, HK_>), g, wg, 0, s, L.k, F, mask, R)
+#define FC2(FX, CS)                                \
+  if (hb && hk) { FC(FX, CS, true, true); }        \
+  else if (hb) { FC(FX, CS, true, false); }        \
+  else if (hk) { FC(FX, CS, false, true); }        \
+  else { FC(FX, CS, false, false); }
   if (fix && cons) {
     FC2(true, true)
   } else if (fix) {
@@ -704,7 +711,7 @@ static void flux_dir(const LaunchCtx &L, const KFields &F, double *const *alfven
   const dim3 g = tile_grid(R), wg(shared || march || pair ? TILE : R.tile);
   const dim3 g2((unsigned)(((2 * R.ntiles + 7) / 8) * 8));
   const bool hb = L.k.iBX >= 0, hk = L.k.iKEL >= 0;
-  const int lim = L.limiter, rs = L.riemann;
+  const int lim = L.limiter, rs = L.riemann, mf = metric_form(L.metric);
 #define FL(LIM, RS, HB_, HK_)                                                                      \
   if (shared)                                                                                     \
     hipLaunchKernelGGL((k_flux_x1s<LIM, RS, HB_, HK_>), g, kTile, 0, s, L.k, F, alfven, R);       \
@@ -713,13 +720,17 @@ static void flux_dir(const LaunchCtx &L, const KFields &F, double *const *alfven
                        alfven, R);                                                                \
   else if (pair)                                                                                  \
     hipLaunchKernelGGL((k_flux_pair<DIR, LIM, RS, HB_, HK_>), g2, kTile, 0, s, L.k, F, alfven, R); \
+  else if (mf == FORM_POLOIDAL)                                                                   \
+    hipLaunchKernelGGL((k_flux<DIR, LIM, RS, HB_, HK_, FORM_POLOIDAL>), g, wg, 0, s, L.k, F, alfven, R); \
+  else if (mf == FORM_FLAT)                                                                       \
+    hipLaunchKernelGGL((k_flux<DIR, LIM, RS, HB_, HK_, FORM_FLAT>), g, wg, 0, s, L.k, F, alfven, R); \
   else                                                                                            \
-    hipLaunchKernelGGL((k_flux<DIR, LIM, RS, HB_, HK_>), g, wg, 0, s, L.k, F, alfven, R)
-#define FL2(LIM, RS)                    \
-  if (hb && hk) FL(LIM, RS, true, true); \
-  else if (hb) FL(LIM, RS, true, false); \
-  else if (hk) FL(LIM, RS, false, true); \
-  else FL(LIM, RS, false, false);
+    hipLaunchKernelGGL((k_flux<DIR, LIM, RS, HB_, HK_, FORM_FULL>), g, wg, 0, s, L.k, F, alfven, R)
+#define FL2(LIM, RS)                         \
+  if (hb && hk) { FL(LIM, RS, true, true); } \
+  else if (hb) { FL(LIM, RS, true, false); } \
+  else if (hk) { FL(LIM, RS, false, true); } \
+  else { FL(LIM, RS, false, false); }
   if (lim == PANGU_LIMITER_PPM4 && rs == PANGU_RIEMANN_LAXF) {
     FL2(PANGU_LIMITER_PPM4, PANGU_RIEMANN_LAXF)
   } else if (lim == PANGU_LIMITER_PPM4) {

@@ -32,42 +32,97 @@ struct Phys {
 __device__ __forceinline__ double kmax(double a, double b) { return (a < b) ? b : a; }
 __device__ __forceinline__ double kmin(double a, double b) { return (b < a) ? b : a; }
 
+// Structure of a metric's tables, fixed by the coordinates (checked for every
+// metric in tests/test_metric_form.py).  A kernel compiled for a form reads
+// only the entries the form leaves open, and drops the terms whose metric
+// factor is exactly zero: adding +-0 leaves a finite sum unchanged (a sum of
+// zeros may differ in sign), so results equal those of the full sums.
+//   FULL      every entry (Cartesian Kerr-Schild); g_{0i} = g_{i0} bit for bit
+//   POLOIDAL  x2 decouples (Kerr-Schild in MKS, Boyer-Lindquist): g_{m2} = 0
+//             for m != 2, g^{02} = 0, and g_{mn} = g_{nm} bit for bit
+//   FLAT      diag(-1, 1, 1, 1): nothing is read
+// The sweeps and FixPrimitive are bound by FP64 issue and by the latency that
+// their few wavefronts leave open (registers), so what a form saves counts
+// twice.  X2 sweep, PPM4 + HLL: 1272 FP64 instructions, 24 table loads and
+// 150 VGPRs for full sums; 1182, 13 and 146 POLOIDAL; 955, none and 116 (four
+// wavefronts instead of three) FLAT without K_e; and 976 to 782 FULL without
+// a field (HB false below).  Per cycle: 3-D torus 256x128x128 4.36 -> 4.19 ms,
+// 2-D torus 512x256 247 -> 233 us, Orszag-Tang 256^2 134 -> 118 us, refined
+// Cartesian Kerr-Schild without a field 458 -> 423 us.
+enum MetricForm { FORM_FULL = 0, FORM_POLOIDAL = 1, FORM_FLAT = 2 };
+
+// Is g_{rc} possibly non-zero?
+template <int MF>
+__host__ __device__ constexpr bool g_open(int r, int c) {
+  return MF == FORM_FULL || r == c || (MF == FORM_POLOIDAL && r != 2 && c != 2);
+}
+// Table slot (4 r + c) that holds g_{rc}: symmetric entries share one.
+template <int MF>
+__host__ __device__ constexpr int g_slot(int r, int c) {
+  return (r > c && (MF != FORM_FULL || c == 0)) ? 4 * c + r : 4 * r + c;
+}
+// Is g^{0m} possibly non-zero?
+template <int MF>
+__host__ __device__ constexpr bool g0_open(int m) {
+  return m == 0 || MF == FORM_FULL || (MF == FORM_POLOIDAL && m != 2);
+}
+
+// g_{rc} x^c over c = C0 .. 3, added in ascending c.
+template <int MF, int C0 = 0>
+__device__ __forceinline__ double lower(const double g[16], int r, const double x[4]) {
+  double v = 0.0;
+  bool first = true;
+#pragma unroll
+  for (int c = C0; c < 4; ++c) {
+    if (!g_open<MF>(r, c)) continue;
+    v = first ? g[4 * r + c] * x[c] : v + g[4 * r + c] * x[c];
+    first = false;
+  }
+  return v;
+}
+
 // Fluid state u^mu, u_mu, b^mu, b_mu, b^2 (state_calculation.h:19-69).
-// g: gcov row-major; gc0: gcon[0][0..3]; alpha = 1/sqrt(-gcon00).
+// g: gcov row-major; gc0: gcon[0][0..3]; alpha = 1/sqrt(-gcon00).  HB false:
+// no magnetic field (b = 0; the other quantities are those of B = 0).
 struct St {
   double ucon[4], ucov[4], bcon[4], bcov[4], bsq;
 };
 
+template <int MF = FORM_FULL, bool HB = true>
 __device__ __forceinline__ void calc_state(const double p[NPRIM], const double g[16],
                                            const double gc0[4], double alpha, St &s) {
-  const double v1 = p[UX1], v2 = p[UX2], v3 = p[UX3];
-  double sq = v1 * g[5] * v1;
-  sq = sq + v1 * g[6] * v2;
-  sq = sq + v1 * g[7] * v3;
-  sq = sq + v2 * g[9] * v1;
-  sq = sq + v2 * g[10] * v2;
-  sq = sq + v2 * g[11] * v3;
-  sq = sq + v3 * g[13] * v1;
-  sq = sq + v3 * g[14] * v2;
-  sq = sq + v3 * g[15] * v3;
+  const double v[3] = {p[UX1], p[UX2], p[UX3]};
+  double sq = 0.0;
+  bool first = true;
+#pragma unroll
+  for (int r = 0; r < 3; ++r)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      if (!g_open<MF>(r + 1, c + 1)) continue;
+      const double t = v[r] * g[4 * (r + 1) + c + 1] * v[c];
+      sq = first ? t : sq + t;
+      first = false;
+    }
   const double lor = sqrt(1.0 + sq);
   s.ucon[0] = lor / alpha;
-  s.ucon[1] = v1 - s.ucon[0] * gc0[1] * alpha * alpha;
-  s.ucon[2] = v2 - s.ucon[0] * gc0[2] * alpha * alpha;
-  s.ucon[3] = v3 - s.ucon[0] * gc0[3] * alpha * alpha;
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-    s.ucov[r] = g[4 * r] * s.ucon[0] + g[4 * r + 1] * s.ucon[1] + g[4 * r + 2] * s.ucon[2] +
-                g[4 * r + 3] * s.ucon[3];
+  for (int c = 1; c < 4; ++c)
+    s.ucon[c] = g0_open<MF>(c) ? v[c - 1] - s.ucon[0] * gc0[c] * alpha * alpha : v[c - 1];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) s.ucov[r] = lower<MF>(g, r, s.ucon);
+  if (!HB) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s.bcon[r] = s.bcov[r] = 0.0;
+    s.bsq = 0.0;
+    return;
+  }
   s.bcon[0] = p[BX1] * s.ucov[1] + p[BX2] * s.ucov[2] + p[BX3] * s.ucov[3];
   const double ru0 = 1.0 / s.ucon[0];
   s.bcon[1] = div_by(p[BX1] + s.bcon[0] * s.ucon[1], s.ucon[0], ru0);
   s.bcon[2] = div_by(p[BX2] + s.bcon[0] * s.ucon[2], s.ucon[0], ru0);
   s.bcon[3] = div_by(p[BX3] + s.bcon[0] * s.ucon[3], s.ucon[0], ru0);
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-    s.bcov[r] = g[4 * r] * s.bcon[0] + g[4 * r + 1] * s.bcon[1] + g[4 * r + 2] * s.bcon[2] +
-                g[4 * r + 3] * s.bcon[3];
+  for (int r = 0; r < 4; ++r) s.bcov[r] = lower<MF>(g, r, s.bcon);
   s.bsq = s.bcon[0] * s.bcov[0] + s.bcon[1] * s.bcov[1] + s.bcon[2] * s.bcov[2] +
           s.bcon[3] * s.bcov[3];
 }
@@ -75,30 +130,30 @@ __device__ __forceinline__ void calc_state(const double p[NPRIM], const double g
 // T^dir_m (energy_momentum_tensor.h:11-29).  The reference's
 // p_tot*(dir==m) term is added only where it is non-zero (adding +0 leaves
 // the sum unchanged).
-template <int DIR>
+template <int DIR, bool HB = true>
 __device__ __forceinline__ double tmunu(const St &s, double etot, double ptot, int m) {
   double v = etot * s.ucon[DIR] * s.ucov[m];
   if (m == DIR) v = v + ptot;
-  return v - s.bcon[DIR] * s.bcov[m];
+  return HB ? v - s.bcon[DIR] * s.bcov[m] : v;
 }
 
 // sqrt|g| * F^dir (contravariant_flux.h:12-39) for every slot of the vector.
-template <int DIR>
+template <int DIR, bool HB = true>
 __device__ __forceinline__ void contravariant_flux(double gamma, const double p[NPRIM], const St &s,
                                                    double sg, double f[NPRIM]) {
   const double pg = (gamma - 1.) * p[ENY];
   const double h = p[RHO] + gamma * p[ENY];
-  const double etot = h + s.bsq;
-  const double ptot = pg + 0.5 * s.bsq;
+  const double etot = HB ? h + s.bsq : h;
+  const double ptot = HB ? pg + 0.5 * s.bsq : pg;
   const double mflux = p[RHO] * s.ucon[DIR];
   f[RHO] = mflux * sg;
-  f[ENY] = (tmunu<DIR>(s, etot, ptot, 0) + mflux) * sg;
-  f[UX1] = tmunu<DIR>(s, etot, ptot, 1) * sg;
-  f[UX2] = tmunu<DIR>(s, etot, ptot, 2) * sg;
-  f[UX3] = tmunu<DIR>(s, etot, ptot, 3) * sg;
-  f[BX1] = (s.bcon[1] * s.ucon[DIR] - s.bcon[DIR] * s.ucon[1]) * sg;
-  f[BX2] = (s.bcon[2] * s.ucon[DIR] - s.bcon[DIR] * s.ucon[2]) * sg;
-  f[BX3] = (s.bcon[3] * s.ucon[DIR] - s.bcon[DIR] * s.ucon[3]) * sg;
+  f[ENY] = (tmunu<DIR, HB>(s, etot, ptot, 0) + mflux) * sg;
+  f[UX1] = tmunu<DIR, HB>(s, etot, ptot, 1) * sg;
+  f[UX2] = tmunu<DIR, HB>(s, etot, ptot, 2) * sg;
+  f[UX3] = tmunu<DIR, HB>(s, etot, ptot, 3) * sg;
+#pragma unroll
+  for (int a = 1; a < 4; ++a)  // the normal field is not transported: b^d u^d - b^d u^d = 0
+    f[BX1 + a - 1] = (!HB || a == DIR) ? 0.0 : (s.bcon[a] * s.ucon[DIR] - s.bcon[DIR] * s.ucon[a]) * sg;
   f[ENT] = (p[ENT] * mflux) * sg;
   f[KEL] = (p[KEL] * mflux) * sg;
 }
@@ -106,21 +161,24 @@ __device__ __forceinline__ void contravariant_flux(double gamma, const double p[
 // Fast magnetosonic speeds along DIR (fast_magnetosonic_speed.h:11-81).  With
 // n_mu = e^DIR and t_mu = e^0 the reference's contractions reduce exactly to
 // n^2 = gcon[DIR][DIR], t^2 = gcon00, n.t = gcon[0][DIR], n.u = u^DIR, t.u = u^0.
-template <int DIR>
+template <int DIR, int MF = FORM_FULL, bool HB = true>
 __device__ __forceinline__ void fast_ms(double gamma, const double p[NPRIM], const St &s,
                                         double gcon00, double gcon0d, double gcondd,
                                         double &vmax, double &vmin) {
   const double h = p[RHO] + gamma * p[ENY];
-  const double htot = s.bsq + h;
-  const double va2 = s.bsq / htot;
   const double cs2 = gamma * (gamma - 1.) * p[ENY] / h;
-  double cf2 = cs2 + va2 - cs2 * va2;
+  double cf2 = cs2;
+  if (HB) {
+    const double htot = s.bsq + h;
+    const double va2 = s.bsq / htot;
+    cf2 = cs2 + va2 - cs2 * va2;
+  }
   if (cf2 < 0.) cf2 = 1e-10;
   if (cf2 > 1.) cf2 = 1.;
   const double nu = s.ucon[DIR], tu = s.ucon[0];
   const double nu2 = nu * nu, tu2 = tu * tu, nutu = nu * tu;
   const double A = tu2 - (gcon00 + tu2) * cf2;
-  const double B = 2. * (nutu - (gcon0d + nutu) * cf2);
+  const double B = 2. * (nutu - (g0_open<MF>(DIR) ? gcon0d + nutu : nutu) * cf2);
   const double C = nu2 - (gcondd + nu2) * cf2;
   double disc = B * B - 4. * A * C;
   if ((disc < 0.0) && (disc > -1.e-10)) {
