@@ -198,7 +198,8 @@ __device__ __forceinline__ void flux_div(const DevBlock &B, const KFields &F0, c
 // without spilling (the field-free ones spill at five and run at four); the
 // kernel is memory bound, so occupancy pays.
 // One cell of k_div_update; the new U also goes to uout (when given).
-template <int MODE, bool SRC, bool HB, bool HK, bool CTF>
+// MF: form of the metric for the source term (FORM_FLAT: no source).
+template <int MODE, int MF, bool HB, bool HK, bool CTF>
 __device__ __forceinline__ void div_update_cell(const KCtx &C, const KFields &F0, const KFields &Finit,
                                                 const KFields &F1, double *const *dudt,
                                                 const double *dt_dev, double beta, double bdt_host,
@@ -230,29 +231,29 @@ __device__ __forceinline__ void div_update_cell(const KCtx &C, const KFields &F0
     for (int q = 0; q < NC; ++q) unew[q] = glb(F1.cons[b * NC + q])[id];
   }
   if (MODE == 1) return;
-  if (SRC && (MODE == 3 || MODE == 4)) {
+  if (MF != FORM_FLAT && (MODE == 3 || MODE == 4)) {
     const DevGeo &G = C.geo[B.geo];
     const int64_t t = cen_index(G, k, j, i);
     CenLoad m;
-    load_cen_state(G, t, m);
+    load_cen_state<MF>(G, t, m);
     double p[NPRIM];
 #pragma unroll
     for (int s = 0; s < NPRIM; ++s) p[s] = 0.0;
 #pragma unroll
     for (int q = 0; q < NC; ++q) p[slot_of<HB, HK>(q)] = glb(F1.prim[b * NC + q])[id];
     St s;
-    calc_state(p, m.g, m.gc0, m.alpha, s);
+    calc_state<MF, HB>(p, m.g, m.gc0, m.alpha, s);
     const double gam = C.ph.gamma;
     const double pg = (gam - 1.) * p[ENY];
     const double h = p[RHO] + gam * p[ENY];
-    const double etot = h + s.bsq, ptot = pg + 0.5 * s.bsq;
+    const double etot = HB ? h + s.bsq : h, ptot = HB ? pg + 0.5 * s.bsq : pg;
     double T[4][4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      T[0][c] = tmunu<0>(s, etot, ptot, c);
-      T[1][c] = tmunu<1>(s, etot, ptot, c);
-      T[2][c] = tmunu<2>(s, etot, ptot, c);
-      T[3][c] = tmunu<3>(s, etot, ptot, c);
+      T[0][c] = tmunu<0, HB>(s, etot, ptot, c);
+      T[1][c] = tmunu<1, HB>(s, etot, ptot, c);
+      T[2][c] = tmunu<2, HB>(s, etot, ptot, c);
+      T[3][c] = tmunu<3, HB>(s, etot, ptot, c);
     }
     // one scalar base for the connection block (40 or 64 slots) and a
     // 32-bit index per slot: per-slot scalar bases would exhaust the scalar
@@ -282,14 +283,14 @@ __device__ __forceinline__ void div_update_cell(const KCtx &C, const KFields &F0
   }
 }
 
-template <int MODE, bool SRC, bool HB, bool HK, bool CTF>
+template <int MODE, int MF, bool HB, bool HK, bool CTF>
 __global__ __launch_bounds__(256, (HB && MODE != 1) ? 5 : 4) void k_div_update(KCtx C, KFields F0, KFields Finit, KFields F1,
                                                     double *const *dudt,
                                                     const double *dt_dev, double beta,
                                                     double bdt_host, Range3 R) {
   int b, k, j, i;
   if (!decode_tile(C, R, b, k, j, i)) return;
-  div_update_cell<MODE, SRC, HB, HK, CTF>(C, F0, Finit, F1, dudt, dt_dev, beta, bdt_host, b, k, j, i,
+  div_update_cell<MODE, MF, HB, HK, CTF>(C, F0, Finit, F1, dudt, dt_dev, beta, bdt_host, b, k, j, i,
                                           nullptr);
 }
 
@@ -297,15 +298,15 @@ __global__ __launch_bounds__(256, (HB && MODE != 1) ? 5 : 4) void k_div_update(K
 // ApplyElectronHeating (electron_heating.cc:66-109) on one recovered cell
 // from its primitives p (rho, u, u~, B and the stale entropy; K_e is not
 // read); the centre metric is loaded here.
-template <bool HB, bool HK>
+template <int MF, bool HB, bool HK>
 __device__ __forceinline__ void heat_vals(const KCtx &C, const KFields &F, const DevGeo &G, int64_t t,
                                           int b, int64_t id, const Arr32<double> *pp,
                                           const double p[NPRIM], const double *ureg = nullptr) {
   constexpr int NC = ncomp<HB, HK>();
   CenLoad m;
-  load_cen_state(G, t, m);
+  load_cen_state<MF>(G, t, m);
   St s;
-  calc_state(p, m.g, m.gc0, m.alpha, s);
+  calc_state<MF, HB>(p, m.g, m.gc0, m.alpha, s);
   const uint32_t id32 = (uint32_t)id;
   // conserved components: from memory, or from registers (ureg, in
   // component order) when the caller has just written them
@@ -322,7 +323,7 @@ __device__ __forceinline__ void heat_vals(const KCtx &C, const KFields &F, const
 }
 
 // The same with the primitives read from memory.
-template <bool HB, bool HK>
+template <int MF, bool HB, bool HK>
 __device__ __forceinline__ void heat_cell(const KCtx &C, const KFields &F, const DevGeo &G, int64_t t,
                                           int b, int64_t id, const Arr32<double> *pp) {
   constexpr int NC = ncomp<HB, HK>();
@@ -331,13 +332,31 @@ __device__ __forceinline__ void heat_cell(const KCtx &C, const KFields &F, const
   for (int s = 0; s < NPRIM; ++s) p[s] = 0.0;
 #pragma unroll
   for (int q = 0; q < NC; ++q) p[slot_of<HB, HK>(q)] = pp[q][id];
-  heat_vals<HB, HK>(C, F, G, t, b, id, pp, p);
+  heat_vals<MF, HB, HK>(C, F, G, t, b, id, pp, p);
+}
+
+// The centre metric the recovery reads, as far as form MF leaves it open
+// (gcon is not symmetric bit for bit, so each open entry is read), sqrt|g|
+// and 1/sqrt(-g^00).
+template <int MF>
+__device__ __forceinline__ void load_cen_metric(const DevGeo &G, int64_t t, CenMetric &m, double &sg,
+                                                double &alpha) {
+  auto comp = [&](int n) { return ldc32(G.cen, (int64_t)n * G.ncen, (uint32_t)t); };
+  double gc0[4];
+  load_metric<MF, CG_GCON, CG_ALPHA>(comp, m.gcov, gc0, alpha);
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      m.gcon[4 * r + c] = MF == FORM_FLAT ? m.gcov[4 * r + c] : g_open<MF>(r, c) ? comp(CG_GCON + 4 * r + c) : 0.0;
+  m.lapse = MF == FORM_FLAT ? 1.0 : comp(CG_LAPSE);
+  sg = MF == FORM_FLAT ? 1.0 : comp(CG_SG);
 }
 
 // Recovery (invertor.cc:184-319) and, when HEAT, ApplyElectronHeating
 // (electron_heating.cc:66-109) on the recovered cell.  REC: 0 chainer,
 // 1 Kastaun, 2 1Dvsq alone, -1 none (heating only).
-template <int REC, bool HB, bool HK, bool HEAT>
+template <int MF, int REC, bool HB, bool HK, bool HEAT>
 __device__ __forceinline__ void recover_cell(const KCtx &C, const KFields &F, const SharedTabs &S, int b,
                                              int k, int j, int i, double x0 = -1.0,
                                              const double *ureg = nullptr) {
@@ -346,7 +365,6 @@ __device__ __forceinline__ void recover_cell(const KCtx &C, const KFields &F, co
   constexpr int NC = ncomp<HB, HK>();
   const DevGeo &G = C.geo[B.geo];
   const int64_t t = cen_index(G, k, j, i);
-  const int64_t ns = G.ncen;
   const Phys &P = C.ph;
   Arr32<double> pp[NC];
 #pragma unroll
@@ -354,21 +372,15 @@ __device__ __forceinline__ void recover_cell(const KCtx &C, const KFields &F, co
   if (REC >= 0) {
     const bool chainer = (REC != 1);
     bool excised = false;
-    if (P.metric == PANGU_METRIC_CKS && ldc32(G.cen, (int64_t)CG_RAD * ns, (uint32_t)t) < P.r_excise) excised = true;
+    if (P.metric == PANGU_METRIC_CKS && ldc32(G.cen, (int64_t)CG_RAD * G.ncen, (uint32_t)t) < P.r_excise) excised = true;
     if (excised) {
       if (chainer && S.flag) glb(S.flag[b])[id] = 0.0;
       if (S.status) glb(S.status[b])[id] = -1;
       if (S.iters) glb(S.iters[b])[id] = 0;
     } else {
       CenMetric m;
-#pragma unroll
-      for (int n = 0; n < 16; ++n) {
-        m.gcov[n] = ldc32(G.cen, (int64_t)(CG_GCOV + n) * ns, (uint32_t)t);
-        m.gcon[n] = ldc32(G.cen, (int64_t)(CG_GCON + n) * ns, (uint32_t)t);
-      }
-      m.lapse = ldc32(G.cen, (int64_t)CG_LAPSE * ns, (uint32_t)t);
-      const double sg = ldc32(G.cen, (int64_t)CG_SG * ns, (uint32_t)t);
-      const double alpha = ldc32(G.cen, (int64_t)CG_ALPHA * ns, (uint32_t)t);
+      double sg, alpha;
+      load_cen_metric<MF>(G, t, m, sg, alpha);
       double U[9], Ph[9], bnew[3] = {0.0, 0.0, 0.0};
       Arr32<double> cons[NC];
 #pragma unroll
@@ -417,22 +429,22 @@ __device__ __forceinline__ void recover_cell(const KCtx &C, const KFields &F, co
       bool write = true;
       if (REC == 1) {
         double mu = 0.0;
-        st = c2p_kastaun(U, Ph, P.gamma, m, it, &mu);
+        st = c2p_kastaun<MF>(U, Ph, P.gamma, m, it, &mu);
         if (S.root) glb(S.root[b])[id] = (st == 0) ? mu : __builtin_nan("");
         itn = it;
         write = (st == 0);
       } else if (REC == 2) {
         // x0 >= 0: the learned start (k_recover_learned_vsq)
-        st = c2p_1dvsq(U, Ph, P.gamma, m, it, x0);
+        st = c2p_1dvsq<MF>(U, Ph, P.gamma, m, it, x0);
         itn = it;
       } else {
-        st = c2p_2d(U, Ph, P.gamma, m, it);
+        st = c2p_2d<MF>(U, Ph, P.gamma, m, it);
         itn = it;
         if (st != 0) {
-          st = c2p_1dvsq(U, Ph, P.gamma, m, it);
+          st = c2p_1dvsq<MF>(U, Ph, P.gamma, m, it);
           itn += it;
           if (st != 0) {
-            st = c2p_1d(U, Ph, P.gamma, m, it);
+            st = c2p_1d<MF>(U, Ph, P.gamma, m, it);
             itn += it;
           }
         }
@@ -477,19 +489,19 @@ __device__ __forceinline__ void recover_cell(const KCtx &C, const KFields &F, co
           hp[BX3] = bnew[2];
         }
         hp[ENT] = pp[ient<HB>()][id];
-        heat_vals<HB, HK>(C, F, G, t, b, id, pp, hp, ureg);
+        heat_vals<MF, HB, HK>(C, F, G, t, b, id, pp, hp, ureg);
         return;
       }
     }
   }
-  if (HEAT && HK) heat_cell<HB, HK>(C, F, G, t, b, id, pp);
+  if (HEAT && HK) heat_cell<MF, HB, HK>(C, F, G, t, b, id, pp);
 }
 
-template <int REC, bool HB, bool HK, bool HEAT>
+template <int MF, int REC, bool HB, bool HK, bool HEAT>
 __global__ __launch_bounds__(256) void k_recover(KCtx C, KFields F, SharedTabs S, Range3 R) {
   int b, k, j, i;
   if (!decode_tile(C, R, b, k, j, i)) return;
-  recover_cell<REC, HB, HK, HEAT>(C, F, S, b, k, j, i);
+  recover_cell<MF, REC, HB, HK, HEAT>(C, F, S, b, k, j, i);
 }
 
 // The update of k_div_update (mode 4: flux divergence, RK update, source)
@@ -499,15 +511,21 @@ __global__ __launch_bounds__(256) void k_recover(KCtx C, KFields F, SharedTabs S
 // across the wavefronts of one launch.  Same operations per cell in the same
 // order: identical results.  Called only when nothing has to run between
 // the two (the stage's exchange runs before).
-template <bool SRC, bool HB, bool HK, bool CTF, int REC, bool HEAT>
+// The metric's form (physics_dev.h) keeps what no cell of a mesh needs out of
+// the registers: MKS with Kastaun and heating 165 -> 127 VGPRs (four
+// wavefronts per SIMD instead of three) and 309 -> 288 loads; per cycle
+// 4.186 -> 4.158 ms on the 3-D torus 256x128x128, 233 -> 227 us on the 2-D
+// torus 512x256, 118 -> 109 us on Orszag-Tang 256^2; the chainer alone on a
+// flat 301x199 plane 15.2 -> 11.0 us.
+template <int MF, bool HB, bool HK, bool CTF, int REC, bool HEAT>
 __global__ __launch_bounds__(256) void k_update_recover(KCtx C, KFields F0, KFields Finit, KFields F1,
                                                         SharedTabs S, const double *dt_dev, double beta,
                                                         double bdt_host, Range3 R) {
   int b, k, j, i;
   if (!decode_tile(C, R, b, k, j, i)) return;
   double u[NPRIM];
-  div_update_cell<4, SRC, HB, HK, CTF>(C, F0, Finit, F1, nullptr, dt_dev, beta, bdt_host, b, k, j, i, u);
-  recover_cell<REC, HB, HK, HEAT>(C, F1, S, b, k, j, i, -1.0, u);
+  div_update_cell<4, MF, HB, HK, CTF>(C, F0, Finit, F1, nullptr, dt_dev, beta, bdt_host, b, k, j, i, u);
+  recover_cell<MF, REC, HB, HK, HEAT>(C, F1, S, b, k, j, i, -1.0, u);
 }
 
 // Persistent form of k_recover: a grid no larger than what the GPU holds
@@ -527,7 +545,7 @@ __global__ __launch_bounds__(256) void k_recover_queue(KCtx C, KFields F, Shared
     __syncthreads();  // every thread has read the tile before the next pull
     if (T >= R.ntiles) break;
     int b, k, j, i;
-    if (decode_tile_at(C, R, T, b, k, j, i)) recover_cell<REC, HB, HK, HEAT>(C, F, S, b, k, j, i);
+    if (decode_tile_at(C, R, T, b, k, j, i)) recover_cell<FORM_FULL, REC, HB, HK, HEAT>(C, F, S, b, k, j, i);
   }
   if (threadIdx.x == 0 && atomicAdd(&queue[1], 1u) == gridDim.x - 1) {
     atomicExch(&queue[0], 0u);
@@ -581,7 +599,7 @@ __global__ __launch_bounds__(256) void k_recover_learned(KCtx C, KFields F, Shar
   int b = 0, k = 0, j = 0, i = 0;
   const bool cell = decode_tile(C, R, b, k, j, i);  // false on the whole workgroup past the range
   if (UPD && cell)
-    div_update_cell<4, UPD == 2, HB, HK, HB>(C, A.F0, A.Finit, F, nullptr, A.dt_dev, A.beta, A.bdt_host, b,
+    div_update_cell<4, UPD == 2 ? FORM_FULL : FORM_FLAT, HB, HK, HB>(C, A.F0, A.Finit, F, nullptr, A.dt_dev, A.beta, A.bdt_host, b,
                                              k, j, i, nullptr);
   const int lane = threadIdx.x & 63;
   constexpr int NC = ncomp<HB, HK>();
@@ -690,11 +708,11 @@ __global__ __launch_bounds__(256) void k_recover_learned(KCtx C, KFields F, Shar
         for (int a = 0; a < 3; ++a) hp[BX1 + a] = bnew[a];
       }
       hp[ENT] = pp[ient<HB>()][id];
-      heat_vals<HB, HK>(C, F, G, t, b, id, pp, hp);
+      heat_vals<FORM_FULL, HB, HK>(C, F, G, t, b, id, pp, hp);
       return;
     }
   }
-  if (HEAT && HK) heat_cell<HB, HK>(C, F, G, t, b, id, pp);
+  if (HEAT && HK) heat_cell<FORM_FULL, HB, HK>(C, F, G, t, b, id, pp);
 }
 
 // The 1Dvsq recovery with the learned start (and, when HEAT, the heating):
@@ -711,7 +729,7 @@ __global__ __launch_bounds__(256) void k_recover_learned_vsq(KCtx C, KFields F, 
   int b = 0, k = 0, j = 0, i = 0;
   const bool cell = decode_tile(C, R, b, k, j, i);  // false on the whole workgroup past the range
   if (UPD && cell)
-    div_update_cell<4, UPD == 2, HB, HK, HB>(C, A.F0, A.Finit, F, nullptr, A.dt_dev, A.beta, A.bdt_host, b,
+    div_update_cell<4, UPD == 2 ? FORM_FULL : FORM_FLAT, HB, HK, HB>(C, A.F0, A.Finit, F, nullptr, A.dt_dev, A.beta, A.bdt_host, b,
                                              k, j, i, nullptr);
   const int lane = threadIdx.x & 63;
   const Phys &P = C.ph;
@@ -746,7 +764,7 @@ __global__ __launch_bounds__(256) void k_recover_learned_vsq(KCtx C, KFields F, 
     }
   }
   if (!cell) return;
-  recover_cell<2, HB, HK, HEAT>(C, F, S, b, k, j, i, x0);
+  recover_cell<FORM_FULL, 2, HB, HK, HEAT>(C, F, S, b, k, j, i, x0);
 }
 
 // ---------------------------------------------------------- FixRecovery
@@ -1144,32 +1162,37 @@ int launch_div_update(const LaunchCtx &L, int mode, const KFields &F0, const KFi
   const bool src = L.metric != PANGU_METRIC_MINKOWSKI;
   // CT fused into the divergence (modes 4 and 5 with a field)
   const bool ctf = ct_fused && hb && (mode == 4 || mode == 5);
-#define DU(M, SR, HB_, HK_, CT_)                                                               \
-  hipLaunchKernelGGL((k_div_update<M, SR, HB_, HK_, CT_>), g, wg, 0, s, L.k, F0, Finit, F1, \
+#define DU(M, MF_, HB_, HK_, CT_)                                                               \
+  hipLaunchKernelGGL((k_div_update<M, MF_, HB_, HK_, CT_>), g, wg, 0, s, L.k, F0, Finit, F1, \
                      dudt, dt_dev, beta, bdt_host, R)
-#define DU2(M, SR)                                      \
-  if (hb && hk) {                                       \
-    if ((M) == 4 && ctf) DU(M, SR, true, true, (M) == 4); \
-    else DU(M, SR, true, true, false);                  \
-  } else if (hb) {                                      \
-    if ((M) == 4 && ctf) DU(M, SR, true, false, (M) == 4); \
-    else DU(M, SR, true, false, false);                 \
-  } else if (hk) DU(M, SR, false, true, false);         \
-  else DU(M, SR, false, false, false);
+#define DU2(M, MF_)                                      \
+  if (hb && hk) {                                        \
+    if ((M) == 4 && ctf) DU(M, MF_, true, true, (M) == 4); \
+    else DU(M, MF_, true, true, false);                  \
+  } else if (hb) {                                       \
+    if ((M) == 4 && ctf) DU(M, MF_, true, false, (M) == 4); \
+    else DU(M, MF_, true, false, false);                 \
+  } else if (hk) DU(M, MF_, false, true, false);         \
+  else DU(M, MF_, false, false, false);
+  const int mf = metric_form(L.metric);  // FORM_FLAT: no source term
   switch (mode) {
-    case 1: DU2(1, false) break;
-    case 2: DU2(2, false) break;
+    case 1: DU2(1, FORM_FLAT) break;
+    case 2: DU2(2, FORM_FLAT) break;
     case 3:
-      if (src) {
-        DU2(3, true)
+      if (mf == FORM_POLOIDAL) {
+        DU2(3, FORM_POLOIDAL)
+      } else if (mf == FORM_FULL) {
+        DU2(3, FORM_FULL)
       }
       break;
-    case 5: DU2(4, false) break;
+    case 5: DU2(4, FORM_FLAT) break;
     default:
-      if (src) {
-        DU2(4, true)
+      if (mf == FORM_POLOIDAL) {
+        DU2(4, FORM_POLOIDAL)
+      } else if (mf == FORM_FULL) {
+        DU2(4, FORM_FULL)
       } else {
-        DU2(4, false)
+        DU2(4, FORM_FLAT)
       }
   }
 #undef DU2
@@ -1216,6 +1239,7 @@ int launch_recover(const LaunchCtx &L, const KFields &F, const SharedTabs &S, in
   const dim3 g = tile_grid(R), wg(R.tile);
   const bool hb = L.k.iBX >= 0, hk = L.k.iKEL >= 0;
   const bool persist = L.persist_recovery && L.queue;
+  const int mf = metric_form(L.metric);
 #define RC(R_, HB_, HK_, HE_)                                                                        \
   if ((R_ == 1 && W && W->kind == 0) || (R_ == 2 && W && W->kind == 1))                              \
     launch_learned<HB_, HK_, HE_>(L, F, S, *W, R, g, wg, s, upd);                                     \
@@ -1223,13 +1247,17 @@ int launch_recover(const LaunchCtx &L, const KFields &F, const SharedTabs &S, in
     hipLaunchKernelGGL((k_recover_queue<R_, HB_, HK_, HE_>),                                          \
                        dim3(resident_groups(k_recover_queue<R_, HB_, HK_, HE_>, R.tile, R.ntiles)), wg, \
                        0, s, L.k, F, S, R, L.queue);                                                  \
+  else if (mf == FORM_POLOIDAL)                                                                       \
+    hipLaunchKernelGGL((k_recover<FORM_POLOIDAL, R_, HB_, HK_, HE_>), g, wg, 0, s, L.k, F, S, R);     \
+  else if (mf == FORM_FLAT)                                                                           \
+    hipLaunchKernelGGL((k_recover<FORM_FLAT, R_, HB_, HK_, HE_>), g, wg, 0, s, L.k, F, S, R);         \
   else                                                                                                \
-    hipLaunchKernelGGL((k_recover<R_, HB_, HK_, HE_>), g, wg, 0, s, L.k, F, S, R)
-#define RC2(R_, HE_)                     \
-  if (hb && hk) RC(R_, true, true, HE_);  \
-  else if (hb) RC(R_, true, false, HE_);  \
-  else if (hk) RC(R_, false, true, HE_);  \
-  else RC(R_, false, false, HE_);
+    hipLaunchKernelGGL((k_recover<FORM_FULL, R_, HB_, HK_, HE_>), g, wg, 0, s, L.k, F, S, R)
+#define RC2(R_, HE_)                          \
+  if (hb && hk) { RC(R_, true, true, HE_); }  \
+  else if (hb) { RC(R_, true, false, HE_); }  \
+  else if (hk) { RC(R_, false, true, HE_); }  \
+  else { RC(R_, false, false, HE_); }
   const bool h = heat && hk;
   if (rec == 0) {
     if (h) { RC2(0, true) } else { RC2(0, false) }
@@ -1257,31 +1285,31 @@ struct URArgs {
   double beta, bdt_host;
   const Range3 &R;
 };
-template <bool SRC, bool HB, bool HK, int REC, bool HEAT>
+template <int MF, bool HB, bool HK, int REC, bool HEAT>
 static void launch_ur(const URArgs &a, dim3 g, dim3 wg, hipStream_t s) {
-  hipLaunchKernelGGL((k_update_recover<SRC, HB, HK, HB, REC, HEAT>), g, wg, 0, s, a.k, a.F0, a.Finit,
+  hipLaunchKernelGGL((k_update_recover<MF, HB, HK, HB, REC, HEAT>), g, wg, 0, s, a.k, a.F0, a.Finit,
                      a.F1, a.S, a.dt_dev, a.beta, a.bdt_host, a.R);
 }
-template <bool SRC, int REC>
+template <int MF, int REC>
 static void launch_ur_fields(const URArgs &a, dim3 g, dim3 wg, hipStream_t s, bool hb, bool hk, bool h) {
   if (!hb)
-    launch_ur<SRC, false, false, REC, false>(a, g, wg, s);
+    launch_ur<MF, false, false, REC, false>(a, g, wg, s);
   else if (h)
-    launch_ur<SRC, true, true, REC, true>(a, g, wg, s);
+    launch_ur<MF, true, true, REC, true>(a, g, wg, s);
   else if (hk)
-    launch_ur<SRC, true, true, REC, false>(a, g, wg, s);
+    launch_ur<MF, true, true, REC, false>(a, g, wg, s);
   else
-    launch_ur<SRC, true, false, REC, false>(a, g, wg, s);
+    launch_ur<MF, true, false, REC, false>(a, g, wg, s);
 }
-template <bool SRC>
+template <int MF>
 static void launch_ur_rec(const URArgs &a, dim3 g, dim3 wg, hipStream_t s, int rec, bool hb, bool hk,
                           bool h) {
   if (rec == 0)
-    launch_ur_fields<SRC, 0>(a, g, wg, s, hb, hk, h);
+    launch_ur_fields<MF, 0>(a, g, wg, s, hb, hk, h);
   else if (rec == 1)
-    launch_ur_fields<SRC, 1>(a, g, wg, s, hb, hk, h);
+    launch_ur_fields<MF, 1>(a, g, wg, s, hb, hk, h);
   else
-    launch_ur_fields<SRC, 2>(a, g, wg, s, hb, hk, h);
+    launch_ur_fields<MF, 2>(a, g, wg, s, hb, hk, h);
 }
 
 int launch_update_recover(const LaunchCtx &L, const KFields &F0, const KFields &Finit,
@@ -1291,13 +1319,15 @@ int launch_update_recover(const LaunchCtx &L, const KFields &F0, const KFields &
   if (R.ntiles == 0) return 0;
   const dim3 g = tile_grid(R), wg(R.tile);
   const bool hb = L.k.iBX >= 0, hk = L.k.iKEL >= 0, h = heat && hk;
-  const bool src = L.metric != PANGU_METRIC_MINKOWSKI;
   if ((hb && !ct_fused) || (!hb && hk) || rec < 0 || rec > 2) return -1;
   const URArgs a{L.k, F0, Finit, F1, S, dt_dev, beta, bdt_host, R};
-  if (src)
-    launch_ur_rec<true>(a, g, wg, s, rec, hb, hk, h);
+  const int mf = metric_form(L.metric);
+  if (mf == FORM_POLOIDAL)
+    launch_ur_rec<FORM_POLOIDAL>(a, g, wg, s, rec, hb, hk, h);
+  else if (mf == FORM_FLAT)
+    launch_ur_rec<FORM_FLAT>(a, g, wg, s, rec, hb, hk, h);
   else
-    launch_ur_rec<false>(a, g, wg, s, rec, hb, hk, h);
+    launch_ur_rec<FORM_FULL>(a, g, wg, s, rec, hb, hk, h);
   TICK("update_recovery");
   return PG_CHECK_LAUNCH();
 }

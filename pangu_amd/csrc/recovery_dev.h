@@ -17,7 +17,9 @@ constexpr double W_TOO_BIG = 1.e20;
 constexpr double UTSQ_TOO_BIG = 1.e20;
 constexpr double FAIL_VAL = 1.e30;
 
-// Metric view for recovery: full gcov and gcon plus sqrt(-1/gcon00).
+// Metric view for recovery: full gcov and gcon plus sqrt(-1/gcon00).  The
+// functions below take the metric's form (physics_dev.h) as a template
+// parameter and do not touch entries the form fixes at zero.
 struct CenMetric {
   double gcov[16], gcon[16], lapse;
 };
@@ -27,6 +29,7 @@ struct Noble {
   double ncov0, Bsq, QdotB, QdotBsq, Qdotn, Qtsq, D;
 };
 
+template <int MF>
 __device__ __forceinline__ void noble_setup(const double U[9], const CenMetric &m, Noble &v) {
   v.Bcon[0] = 0.;
   v.Bcon[1] = U[BX1];
@@ -38,20 +41,17 @@ __device__ __forceinline__ void noble_setup(const double U[9], const CenMetric &
   v.Qcov[3] = U[UX3];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    v.Bcov[r] = m.gcov[4 * r] * v.Bcon[0] + m.gcov[4 * r + 1] * v.Bcon[1] +
-                m.gcov[4 * r + 2] * v.Bcon[2] + m.gcov[4 * r + 3] * v.Bcon[3];
-    v.Qcon[r] = m.gcon[4 * r] * v.Qcov[0] + m.gcon[4 * r + 1] * v.Qcov[1] +
-                m.gcon[4 * r + 2] * v.Qcov[2] + m.gcon[4 * r + 3] * v.Qcov[3];
+    v.Bcov[r] = lower<MF, 1>(m.gcov, r, v.Bcon);  // B^0 = 0
+    v.Qcon[r] = lower<MF>(m.gcon, r, v.Qcov);
   }
   v.Bsq = v.Bcon[1] * v.Bcov[1] + v.Bcon[2] * v.Bcov[2] + v.Bcon[3] * v.Bcov[3];
-  const double qb = v.Qcov[0] * v.Bcon[0] + v.Qcov[1] * v.Bcon[1] + v.Qcov[2] * v.Bcon[2] +
-                    v.Qcov[3] * v.Bcon[3];
+  const double qb = v.Qcov[1] * v.Bcon[1] + v.Qcov[2] * v.Bcon[2] + v.Qcov[3] * v.Bcon[3];
   v.QdotB = qb;
   v.QdotBsq = qb * qb;
   // n_mu = (-lapse, 0, 0, 0): n^mu = gcon[mu][0] * (-lapse)
   v.ncov0 = -m.lapse;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) v.ncon[r] = m.gcon[4 * r] * v.ncov0;
+  for (int r = 0; r < 4; ++r) v.ncon[r] = g_open<MF>(r, 0) ? m.gcon[4 * r] * v.ncov0 : 0.0;
   v.Qdotn = v.Qcon[0] * v.ncov0;
   const double qsq = v.Qcov[0] * v.Qcon[0] + v.Qcov[1] * v.Qcon[1] + v.Qcov[2] * v.Qcon[2] +
                      v.Qcov[3] * v.Qcon[3];
@@ -59,22 +59,25 @@ __device__ __forceinline__ void noble_setup(const double U[9], const CenMetric &
   v.D = U[RHO];
 }
 
+template <int MF>
 __device__ __forceinline__ bool noble_utsq(const double p[9], const CenMetric &m, double &out) {
   double u = 0.;
 #pragma unroll
   for (int i = 1; i < 4; i++)
 #pragma unroll
-    for (int j = 1; j < 4; j++) u += m.gcov[4 * i + j] * p[UX1 + i - 1] * p[UX1 + j - 1];
+    for (int j = 1; j < 4; j++)
+      if (g_open<MF>(i, j)) u += m.gcov[4 * i + j] * p[UX1 + i - 1] * p[UX1 + j - 1];
   if ((u < 0.) && (fabs(u) < 1.0e-13)) u = fabs(u);
   if (u < 0. || u > UTSQ_TOO_BIG) return false;
   out = u;
   return true;
 }
 
+template <int MF>
 __device__ __forceinline__ void noble_velocity(const Noble &v, double W, double Gamma, double p[9]) {
 #pragma unroll
   for (int i = 1; i < 4; i++) {
-    const double qt = v.Qcon[i] + v.ncon[i] * v.Qdotn;
+    const double qt = g_open<MF>(i, 0) ? v.Qcon[i] + v.ncon[i] * v.Qdotn : v.Qcon[i];
     p[UX1 + i - 1] = Gamma / (W + v.Bsq) * (qt + v.QdotB * v.Bcon[i] / W);
   }
 }
@@ -97,12 +100,13 @@ __device__ __forceinline__ double vsq_of_w(double Bsq, double QdotBsq, double Qt
 
 // ------------------------------------------------- 2D (W, v^2) Newton scheme
 // scheme_2d.h:99-404.
+template <int MF = FORM_FULL>
 __device__ int c2p_2d(const double U[9], double p[9], double gamma, const CenMetric &m, int &iters) {
   iters = 0;
   Noble v;
-  noble_setup(U, m, v);
+  noble_setup<MF>(U, m, v);
   double utsq;
-  if (!noble_utsq(p, m, utsq)) return 2;
+  if (!noble_utsq<MF>(p, m, utsq)) return 2;
   const double gammasq = 1. + utsq;
   double Gamma = sqrt(gammasq);
   double rho0 = v.D / Gamma;
@@ -179,7 +183,7 @@ __device__ int c2p_2d(const double U[9], double p[9], double gamma, const CenMet
   if ((rho0 <= 0.) || (uu <= 0.)) return 5;
   p[RHO] = rho0;
   p[ENY] = uu;
-  noble_velocity(v, W, Gamma, p);
+  noble_velocity<MF>(v, W, Gamma, p);
   return 0;
 }
 
@@ -202,7 +206,7 @@ __device__ __forceinline__ double w_of_vsq(double D, double K, double vsq, doubl
 __device__ inline double vsq_residual(const double U[9], const CenMetric &m, double K, double gamma,
                                       double x, double *scale) {
   Noble v;
-  noble_setup(U, m, v);
+  noble_setup<FORM_FULL>(U, m, v);
   double pr, rho, uu;
   const double W = w_of_vsq(v.D, K, x, gamma, pr, rho, uu);
   const double fact = v.Bsq + W;
@@ -219,18 +223,19 @@ __device__ inline double vsq_residual(const double U[9], const CenMetric &m, dou
 // same arguments give the same bits, and each evaluation is a pow, which
 // bounds this scheme (n + 1 of them for n steps; evaluating afresh at the top
 // of every step and after the last takes 2 n + 1).
+template <int MF = FORM_FULL>
 __device__ int c2p_1dvsq(const double U[9], double p[9], double gamma, const CenMetric &m,
                          int &iters, double x0 = -1.0) {
   iters = 0;
   const double K = p[ENT];
   Noble v;
-  noble_setup(U, m, v);
+  noble_setup<MF>(U, m, v);
   double x;
   if (x0 >= 0.0) {
     x = x0;
   } else {
     double utsq;
-    if (!noble_utsq(p, m, utsq)) return 2;
+    if (!noble_utsq<MF>(p, m, utsq)) return 2;
     const double gammasq = 1. + utsq;
     x = 1. - 1. / gammasq;
   }
@@ -283,19 +288,20 @@ __device__ int c2p_1dvsq(const double U[9], double p[9], double gamma, const Cen
   if ((rho <= 0.) || (uu <= 0.)) return 5;
   p[RHO] = rho;
   p[ENY] = uu;
-  noble_velocity(v, W, Gamma, p);
+  noble_velocity<MF>(v, W, Gamma, p);
   return 0;
 }
 
 // --------------------------------------------------- 1D W isentropic scheme
 // scheme_1d.h:196-568 with func_1d_orig2.
+template <int MF = FORM_FULL>
 __device__ int c2p_1d(const double U[9], double p[9], double gamma, const CenMetric &m, int &iters) {
   iters = 0;
   const double K = p[ENT];
   Noble v;
-  noble_setup(U, m, v);
+  noble_setup<MF>(U, m, v);
   double utsq;
-  if (!noble_utsq(p, m, utsq)) return 2;
+  if (!noble_utsq<MF>(p, m, utsq)) return 2;
   const double uvsq = 1. + utsq;
   double Gamma = sqrt(uvsq);
   double rho0 = v.D / Gamma;
@@ -362,7 +368,7 @@ __device__ int c2p_1d(const double U[9], double p[9], double gamma, const CenMet
   if ((rho0 <= 0.) || (uu <= 0.)) return 5;
   p[RHO] = rho0;
   p[ENY] = uu;
-  noble_velocity(v, W, Gamma, p);
+  noble_velocity<MF>(v, W, Gamma, p);
   return 0;
 }
 
@@ -396,34 +402,59 @@ struct KastaunIn {
 };
 
 // Returns 0, or 1..4 for an invalid metric, D, tau or S/B invariants.
+template <int MF = FORM_FULL>
 __device__ __forceinline__ int kastaun_setup(const double U[9], const CenMetric &m, KastaunIn &k) {
   const double g0 = m.gcov[5], g1 = m.gcov[6], g2 = m.gcov[7], g3 = m.gcov[10], g4 = m.gcov[11],
                g5 = m.gcov[15];
-  const double det = g0 * g3 * g5 + 2.0 * g1 * g2 * g4 - g0 * g4 * g4 - g1 * g1 * g5 - g2 * g2 * g3;
-  if (!(det > 0.0) || !isfinite(det)) return 1;
-  const double idet = 1.0 / det;
-  const double i0 = (g3 * g5 - g4 * g4) * idet, i1 = (g2 * g4 - g1 * g5) * idet,
-               i2 = (g1 * g4 - g2 * g3) * idet, i3 = (g0 * g5 - g2 * g2) * idet,
-               i4 = (g1 * g2 - g0 * g4) * idet, i5 = (g0 * g3 - g1 * g1) * idet;
+  double i0 = 1.0, i1 = 0.0, i2 = 0.0, i3 = 1.0, i4 = 0.0, i5 = 1.0;
+  if (MF != FORM_FLAT) {
+    double det;
+    if (MF == FORM_POLOIDAL)
+      det = g0 * g3 * g5 - g2 * g2 * g3;
+    else
+      det = g0 * g3 * g5 + 2.0 * g1 * g2 * g4 - g0 * g4 * g4 - g1 * g1 * g5 - g2 * g2 * g3;
+    if (!(det > 0.0) || !isfinite(det)) return 1;
+    const double idet = 1.0 / det;
+    if (MF == FORM_POLOIDAL) {
+      i0 = (g3 * g5) * idet;
+      i2 = -(g2 * g3) * idet;
+      i3 = (g0 * g5 - g2 * g2) * idet;
+      i5 = (g0 * g3) * idet;
+    } else {
+      i0 = (g3 * g5 - g4 * g4) * idet;
+      i1 = (g2 * g4 - g1 * g5) * idet;
+      i2 = (g1 * g4 - g2 * g3) * idet;
+      i3 = (g0 * g5 - g2 * g2) * idet;
+      i4 = (g1 * g2 - g0 * g4) * idet;
+      i5 = (g0 * g3 - g1 * g1) * idet;
+    }
+  }
   const double D = U[RHO];
   if (!(D > 0.0) || !isfinite(D)) return 2;
   const double ncov0 = -m.lapse;
-  const double Qcon0 =
-      m.gcon[0] * U[ENY] + m.gcon[1] * U[UX1] + m.gcon[2] * U[UX2] + m.gcon[3] * U[UX3];
+  const double Qcov[4] = {U[ENY], U[UX1], U[UX2], U[UX3]};
+  const double Qcon0 = lower<MF>(m.gcon, 0, Qcov);
   const double Qdotn = Qcon0 * ncov0;
   const double tau = -Qdotn - D;
   if (!isfinite(tau)) return 3;
   const double S0 = U[UX1], S1 = U[UX2], S2 = U[UX3];
-  k.Su[0] = i0 * S0 + i1 * S1 + i2 * S2;
-  k.Su[1] = i1 * S0 + i3 * S1 + i4 * S2;
-  k.Su[2] = i2 * S0 + i4 * S1 + i5 * S2;
+  if (MF == FORM_FULL) {
+    k.Su[0] = i0 * S0 + i1 * S1 + i2 * S2;
+    k.Su[1] = i1 * S0 + i3 * S1 + i4 * S2;
+    k.Su[2] = i2 * S0 + i4 * S1 + i5 * S2;
+  } else {
+    k.Su[0] = MF == FORM_FLAT ? S0 : i0 * S0 + i2 * S2;
+    k.Su[1] = MF == FORM_FLAT ? S1 : i3 * S1;
+    k.Su[2] = MF == FORM_FLAT ? S2 : i2 * S0 + i5 * S2;
+  }
   const double B0 = U[BX1], B1 = U[BX2], B2 = U[BX3];
   k.B[0] = B0;
   k.B[1] = B1;
   k.B[2] = B2;
-  const double Bd0 = g0 * B0 + g1 * B1 + g2 * B2;
-  const double Bd1 = g1 * B0 + g3 * B1 + g4 * B2;
-  const double Bd2 = g2 * B0 + g4 * B1 + g5 * B2;
+  const double Bu[4] = {0.0, B0, B1, B2};
+  const double Bd0 = lower<MF, 1>(m.gcov, 1, Bu);
+  const double Bd1 = lower<MF, 1>(m.gcov, 2, Bu);
+  const double Bd2 = lower<MF, 1>(m.gcov, 3, Bu);
   const double Bsq = B0 * Bd0 + B1 * Bd1 + B2 * Bd2;
   const double Ssq = k.Su[0] * S0 + k.Su[1] * S1 + k.Su[2] * S2;
   const double SdotB = B0 * S0 + B1 * S1 + B2 * S2;
@@ -546,11 +577,12 @@ __device__ inline void c2p_features(const KastaunIn &k, float f[5]) {
 // scheme_kastaun.h:110-259: Illinois false position on [0,1].  Status 0,
 // 1..4 from the setup, 101..104 from the root search, 5..6 from the
 // reconstruction.  mu_out (optional) receives the root.
+template <int MF = FORM_FULL>
 __device__ int c2p_kastaun(const double U[9], double p[9], double gamma, const CenMetric &m,
                            int &iters, double *mu_out = nullptr) {
   iters = 0;
   KastaunIn k;
-  if (int e = kastaun_setup(U, m, k)) return e;
+  if (int e = kastaun_setup<MF>(U, m, k)) return e;
   double mu;
   const int rs = kastaun_solve(k, gamma, 0.0, 1.0, mu, iters);
   if (rs != 0) return 100 + rs;
