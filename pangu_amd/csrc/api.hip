@@ -564,20 +564,22 @@ static int build_tables(pangu_ctx *c) {
     planes[b] = H.e[2] - H.s[2] + 1;
   }
   if (!r) r = make_items(c, L.ghosts, ghosts);
-  for (int d = 0; d < 3 && !r; ++d) {
-    std::vector<int64_t> slab(c->nblocks, 0);
-    for (int b = 0; b < c->nblocks; ++b) {
-      const HostBlock &H = c->hb[b];
-      const pangu_config &cfg = c->mcfg[c->bmesh[b]];
+  // boundary slabs: both sides of every dim in which a block touches a
+  // physical face (as DevBlock::bcf says, k_bc)
+  std::vector<int64_t> slab(c->nblocks, 0);
+  for (int b = 0; b < c->nblocks; ++b) {
+    const HostBlock &H = c->hb[b];
+    const pangu_config &cfg = c->mcfg[c->bmesh[b]];
+    for (int d = 0; d < 3; ++d) {
       if (H.n[d] == 1) continue;
       const bool lo = H.lx[d] == 0 && cfg.bc[d][0] != PANGU_BC_PERIODIC;
-      const bool hi = H.lx[d] == cfg.nb[d] - 1 && cfg.bc[d][1] != PANGU_BC_PERIODIC;
+      const bool hi = (int64_t)H.lx[d] == ((int64_t)cfg.nb[d] << H.level) - 1 && cfg.bc[d][1] != PANGU_BC_PERIODIC;
       if (!lo && !hi) continue;
       const int other = d == 0 ? H.n[1] * H.n[2] : (d == 1 ? H.n[0] * H.n[2] : H.n[0] * H.n[1]);
-      slab[b] = 2 * (int64_t)H.s[d] * other;
+      slab[b] += 2 * (int64_t)H.s[d] * other;
     }
-    r = make_items(c, L.bcs[d], slab);
   }
+  if (!r) r = make_items(c, L.bcs, slab);
   if (r) return r;
   // interior planes: one entry per (block, k) plane (dt reduction, FixRecovery)
   const int *pb = nullptr, *pf = nullptr;

@@ -123,7 +123,7 @@ struct LaunchCtx {
   Range3 interior, entire, face[3], ct;
   Range3 fixx1;  // the entire range in runs of 248 cells (k_fix_flux_x1)
   Range3 x1cells;                  // cell range of the shared-reconstruction X1 sweep
-  Items ghosts, bcs[3];
+  Items ghosts, bcs;
   int order[PANGU_KF_COUNT] = {};  // tile order per kernel family (PANGU_ORDER_*)
   int split_source = 0;            // fused stage: source term in a kernel of its own
   int fuse_ct = 1;                 // fused stage: CT face fluxes formed in the update kernel

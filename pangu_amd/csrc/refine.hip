@@ -57,22 +57,62 @@ __device__ __forceinline__ double minmod(double a, double b) {
   return 0.0;
 }
 
+template <int NP>
 __global__ __launch_bounds__(256) void k_xfill(KCtx C, KFields F, double *const *flag,
                                                const XFill *tab, int n) {
   const int e = (int)(blockIdx.x * 256 + threadIdx.x);
   if (e >= n) return;
   const XFill X = tab[e];
-  const int np = C.np;
+  // every pointer and value is loaded before the first store (a store may
+  // alias the pointer tables and the other arrays)
+  double *to[NP];
+  double v[NP], fl = 0.0;
+#pragma unroll
+  for (int q = 0; q < NP; ++q) to[q] = F.prim[X.db * NP + q];
   if (!X.mean) {
-    for (int q = 0; q < np; ++q) glb(F.prim[X.db * np + q])[X.dst] = glb(F.prim[X.sb * np + q])[X.src];
-    if (flag) glb(flag[X.db])[X.dst] = glb(flag[X.sb])[X.src];
-    return;
+#pragma unroll
+    for (int q = 0; q < NP; ++q) v[q] = glb(F.prim[X.sb * NP + q])[X.src];
+    if (flag) fl = glb(flag[X.sb])[X.src];
+  } else {
+    const DevBlock &S = C.blk[X.sb];
+    const int dim = block_dim(S), sj = S.n[0], sk = S.n[0] * S.n[1];
+#pragma unroll
+    for (int q = 0; q < NP; ++q) v[q] = fine_mean(glb(F.prim[X.sb * NP + q]), X.src, dim, sj, sk);
+    if (flag) fl = fine_min(glb(flag[X.sb]), X.src, dim, sj, sk);
   }
-  const DevBlock &S = C.blk[X.sb];
-  const int dim = block_dim(S), sj = S.n[0], sk = S.n[0] * S.n[1];
-  for (int q = 0; q < np; ++q)
-    glb(F.prim[X.db * np + q])[X.dst] = fine_mean(glb(F.prim[X.sb * np + q]), X.src, dim, sj, sk);
-  if (flag) glb(flag[X.db])[X.dst] = fine_min(glb(flag[X.sb]), X.src, dim, sj, sk);
+  double *const tf = flag ? flag[X.db] : nullptr;
+#pragma unroll
+  for (int q = 0; q < NP; ++q) glb(to[q])[X.dst] = v[q];
+  if (flag) glb(tf)[X.dst] = fl;
+}
+
+// One component of one coarse cell prolongated into the ghosts it covers,
+// with the dimension fixed so that the stencil lives in registers and its
+// coarse gathers are in flight together.
+template <int DIM>
+__device__ __forceinline__ void prolong(const KFields &F, const XProl &X, int np, int q, int sj, int sk) {
+  constexpr int NS = 1 + 2 * DIM;
+  double *const ownp = F.prim[X.b * np + q];
+  const auto own = glb(ownp);
+  double v[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    v[s] = 0.0;
+    if (X.sb[s] >= 0) v[s] = glb(F.prim[X.sb[s] * np + q])[X.sc[s]];
+  }
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+    if (X.sb[s] < 0) v[s] = fine_mean(own, X.sc[s], DIM, sj, sk);
+  double sl[DIM];
+#pragma unroll
+  for (int d = 0; d < DIM; ++d) sl[d] = 0.25 * minmod(v[0] - v[1 + 2 * d], v[2 + 2 * d] - v[0]);
+#pragma unroll
+  for (int c = 0; c < (1 << DIM); ++c) {
+    double w = v[0];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) w = ((c >> d) & 1) ? w + sl[d] : w - sl[d];
+    if ((X.mask >> c) & 1) own[X.base + (c & 1) + ((c >> 1) & 1) * sj + ((c >> 2) & 1) * sk] = w;
+  }
 }
 
 __global__ __launch_bounds__(256) void k_xprol(KCtx C, KFields F, double *const *flag,
@@ -82,7 +122,7 @@ __global__ __launch_bounds__(256) void k_xprol(KCtx C, KFields F, double *const 
   const XProl X = tab[e];
   const DevBlock &B = C.blk[X.b];
   const int dim = block_dim(B), sj = B.n[0], sk = B.n[0] * B.n[1];
-  const int np = C.np, ns = 1 + 2 * dim, q = (int)blockIdx.y;
+  const int np = C.np, q = (int)blockIdx.y;
   if (q == np) {  // the flag row (only when flag != null): copy of the coarse value
     const double f = glb(flag[X.sb[0]])[X.sc[0]];
     const auto out = glb(flag[X.b]);
@@ -90,18 +130,12 @@ __global__ __launch_bounds__(256) void k_xprol(KCtx C, KFields F, double *const 
       if ((X.mask >> c) & 1) out[X.base + (c & 1) + ((c >> 1) & 1) * sj + ((c >> 2) & 1) * sk] = f;
     return;
   }
-  const auto own = glb(F.prim[X.b * np + q]);
-  double v[7];
-  for (int s = 0; s < ns; ++s)
-    v[s] = X.sb[s] >= 0 ? glb(F.prim[X.sb[s] * np + q])[X.sc[s]] : fine_mean(own, X.sc[s], dim, sj, sk);
-  double sl[3];
-  for (int d = 0; d < dim; ++d) sl[d] = 0.25 * minmod(v[0] - v[1 + 2 * d], v[2 + 2 * d] - v[0]);
-  for (int c = 0; c < (1 << dim); ++c) {
-    if (!((X.mask >> c) & 1)) continue;
-    double w = v[0];
-    for (int d = 0; d < dim; ++d) w = ((c >> d) & 1) ? w + sl[d] : w - sl[d];
-    own[X.base + (c & 1) + ((c >> 1) & 1) * sj + ((c >> 2) & 1) * sk] = w;
-  }
+  if (dim == 3)
+    prolong<3>(F, X, np, q, sj, sk);
+  else if (dim == 2)
+    prolong<2>(F, X, np, q, sj, sk);
+  else
+    prolong<1>(F, X, np, q, sj, sk);
 }
 
 __global__ __launch_bounds__(256) void k_flux_correct(KCtx C, KFields F, const XFlux *tab, int n) {
@@ -128,8 +162,13 @@ __global__ __launch_bounds__(256) void k_flux_correct(KCtx C, KFields F, const X
 int launch_exchange_ml(const LaunchCtx &L, const KFields &F, double *const *flag, hipStream_t s) {
   const MultiLevel &M = L.ml;
   if (M.nfill > 0) {
-    hipLaunchKernelGGL(k_xfill, dim3((M.nfill + 255) / 256), dim3(256), 0, s, L.k, F, flag, M.fill,
-                       M.nfill);
+    const dim3 g((M.nfill + 255) / 256), wg(256);
+    switch (L.k.np) {  // packed components: 6, and 3 more with a field, 1 more with K_e
+      case 6: hipLaunchKernelGGL(k_xfill<6>, g, wg, 0, s, L.k, F, flag, M.fill, M.nfill); break;
+      case 7: hipLaunchKernelGGL(k_xfill<7>, g, wg, 0, s, L.k, F, flag, M.fill, M.nfill); break;
+      case 9: hipLaunchKernelGGL(k_xfill<9>, g, wg, 0, s, L.k, F, flag, M.fill, M.nfill); break;
+      default: hipLaunchKernelGGL(k_xfill<10>, g, wg, 0, s, L.k, F, flag, M.fill, M.nfill);
+    }
     if (L.clock) (void)L.clock->mark("exchange_fill", s);
   }
   if (M.nprol > 0) {
