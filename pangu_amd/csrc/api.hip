@@ -1171,12 +1171,20 @@ int pangu_stage(pangu_ctx *c, int md_init, int md0, int md1, double beta, double
   // FixPrimitive + conservative and the X1 sweep in one kernel (the plain
   // per-face X1 form only)
   const bool fuse_fx = c->L.fuse_fix_x1 && !c->L.share_x1 && !(c->L.pair_flux & 1);
+  // For the same reason the exchange may share the sweeps' launch, which
+  // saves its own and hides its memory traffic behind their arithmetic.
+  const bool ride = exchange_after == 0 && md1 != md0 && !overlap && !fuse_fx && exchange_rides(c->L);
   if (fuse_fx) {
     LCHK(c, launch_fix_flux_x1(c->L, f0, c->dmask, c->dalfven, s));
     LCHK(c, launch_fluxes_23(c->L, f0, c->dalfven, s));
   } else {
     LCHK(c, launch_fix_cons(c->L, f0, c->dmask, true, true, s));
-    LCHK(c, launch_fluxes(c->L, f0, c->dalfven, s));
+    if (ride) {
+      const ExchangeArgs ex{f1, c->dflag, c->dnbr};
+      LCHK(c, launch_sweeps(c->L, f0, c->dalfven, &ex, s));
+    } else {
+      LCHK(c, launch_fluxes(c->L, f0, c->dalfven, s));
+    }
   }
   // With fuse_ct the update kernel forms the edge EMFs and the CT face B
   // fluxes itself, so no CT kernel runs: the flux arrays keep the Riemann B
@@ -1197,7 +1205,7 @@ int pangu_stage(pangu_ctx *c, int md_init, int md0, int md1, double beta, double
   if (fuse_ur) {
     if (overlap)
       HIPCHK(c, hipStreamWaitEvent(s, c->ev_join, 0));
-    else if (exchange_after == 0)
+    else if (exchange_after == 0 && !ride)
       LCHK(c, exchange(c, f1, s));
     if (Wl) {
       // the learned kernel of the scheme, with the update run first
@@ -1221,7 +1229,7 @@ int pangu_stage(pangu_ctx *c, int md_init, int md0, int md1, double beta, double
   if (!fuse_ur) {
     if (overlap)
       HIPCHK(c, hipStreamWaitEvent(s, c->ev_join, 0));
-    else if (exchange_after == 0)
+    else if (exchange_after == 0 && !ride)
       LCHK(c, exchange(c, f1, s));
     LCHK(c, launch_recover(c->L, f1, shared_tabs(c), c->cfg.recovery, c->cfg.enable_heating != 0, Wl,
                            s));

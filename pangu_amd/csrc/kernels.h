@@ -165,7 +165,27 @@ void set_kernel_clock(pangu_ctx *c, KernelClock *clock);
 
 int launch_fix_cons(const LaunchCtx &L, const KFields &F, uint8_t *const *mask, bool fix, bool cons,
                     hipStream_t s);
+// The sweeps along every active direction, in one launch where sweeps_merge
+// holds (sweeps.hip).
 int launch_fluxes(const LaunchCtx &L, const KFields &F, double *const *alfven, hipStream_t s);
+// Do all directions run the one-lane sweep in one tile size (and untimed: a
+// kernel clock times each direction by itself)?
+bool sweeps_merge(const LaunchCtx &L);
+// A same-level ghost exchange to run beside the sweeps: container, flag and
+// neighbour table of launch_exchange.
+struct ExchangeArgs {
+  KFields F;
+  double *const *flag;
+  const int *nbr;
+};
+// The merged launch, with an exchange of another container than F's or none
+// (needs 256-cell tiles: exchange_rides).
+int launch_sweeps(const LaunchCtx &L, const KFields &F, double *const *alfven, const ExchangeArgs *ex,
+                  hipStream_t s);
+inline bool exchange_rides(const LaunchCtx &L) {
+  const int t = L.tile[PANGU_KF_FLUX_X1];
+  return sweeps_merge(L) && !L.ml.on && (t == 0 || t == 256);
+}
 // Edge EMFs, then the CT face B fluxes (the task-level ConstraintedTransport).
 int launch_ct(const LaunchCtx &L, const KFields &F, double *const *emf, hipStream_t s);
 // mode: 1 divergence -> dudt, 2 update from dudt, 3 source only, 4 fused

@@ -227,8 +227,8 @@ __device__ __forceinline__ void recon_ppm4(double qm2, double qm1, double q0, do
     ql = q0;
     qr = q0;
   } else {
-    if (fabs(qc) >= 2.0 * fabs(qd)) qr = q0 - 2.0 * qd;
-    if (fabs(qd) >= 2.0 * fabs(qc)) ql = q0 - 2.0 * qc;
+    if (__builtin_expect(fabs(qc) >= 2.0 * fabs(qd), 0)) qr = q0 - 2.0 * qd;
+    if (__builtin_expect(fabs(qd) >= 2.0 * fabs(qc), 0)) ql = q0 - 2.0 * qc;
   }
   ql_ip1 = qr;
   qr_i = ql;

@@ -194,10 +194,13 @@ __device__ __forceinline__ bool decode_march(const KCtx &C, const Range3 &R, int
   return true;
 }
 
-// Block and item index of this thread in an item launch.
+// Block and item index of this thread in tile T of an item launch.
+__device__ __forceinline__ void decode_item_at(const Items &I, int T, int &b, int &item) {
+  b = I.tblock[T];
+  item = (T - I.tfirst[b]) * TILE + (int)threadIdx.x;
+}
 __device__ __forceinline__ void decode_item(const Items &I, int &b, int &item) {
-  b = I.tblock[blockIdx.x];
-  item = ((int)blockIdx.x - I.tfirst[b]) * TILE + (int)threadIdx.x;
+  decode_item_at(I, (int)blockIdx.x, b, item);
 }
 
 }  // namespace pangu
