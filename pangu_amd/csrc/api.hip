@@ -596,14 +596,19 @@ static int build_tables(pangu_ctx *c) {
     const HostBlock &H = c->hb[b];
     maxplane = std::max(maxplane, (int64_t)(H.e[0] - H.s[0] + 1) * (H.e[1] - H.s[1] + 1));
   }
-  L.k.dtper = dt_per_thread(maxplane);
-  const int64_t chunk = 256 * (int64_t)L.k.dtper;
   std::vector<int64_t> dtitems(c->nblocks);
-  for (int b = 0; b < c->nblocks; ++b) {
-    const HostBlock &H = c->hb[b];
-    const int64_t plane = (int64_t)(H.e[0] - H.s[0] + 1) * (H.e[1] - H.s[1] + 1);
-    dtitems[b] = planes[b] * ((plane + chunk - 1) / chunk);
+  for (L.k.dtper = dt_per_thread(maxplane);; L.k.dtper /= 4) {
+    const int64_t chunk = 256 * (int64_t)L.k.dtper;
+    int64_t total = 0;
+    for (int b = 0; b < c->nblocks; ++b) {
+      const HostBlock &H = c->hb[b];
+      const int64_t plane = (int64_t)(H.e[0] - H.s[0] + 1) * (H.e[1] - H.s[1] + 1);
+      dtitems[b] = planes[b] * ((plane + chunk - 1) / chunk);
+      total += dtitems[b];
+    }
+    if (L.k.dtper == 1 || total >= kDtItems) break;
   }
+  for (int m = 0; m < c->nmesh; ++m) L.maxblocks = std::max(L.maxblocks, c->mfirst[m + 1] - c->mfirst[m]);
   const int *db = nullptr, *dfi = nullptr;
   int nd = 0;
   if (int e = upload_tiles(c, dtitems, &db, &dfi, &nd)) return e;

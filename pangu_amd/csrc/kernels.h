@@ -113,13 +113,21 @@ struct MultiLevel {
 // scans 256 * dt_per_thread(plane) cells of a plane, at most 4096 (a 64x64
 // plane is one item, a 512x256 plane 32), with that many loads per thread
 // in flight together; a mesh of small planes keeps the register count (and
-// the workgroups resident) of one load per thread.
+// the workgroups resident) of one load per thread.  build_tables divides it
+// further while the mesh has fewer than kDtItems items.
 inline int dt_per_thread(int64_t plane) { return plane <= 256 ? 1 : (plane <= 1024 ? 4 : 16); }
+// (16 workgroups with 48 loads per thread scanned a 256^2 block in 9.9 us;
+// with the final kernel's lanes sharing a block's items, cycles went
+// Orszag-Tang 256^2 84.5 -> 79.2 us, 2-D torus 512x256 190 -> 182 us, refined
+// 358 -> 354 us, 3-D torus 256x128x128, whose items stay as they were, 3.98 ->
+// 3.93 ms.)
+constexpr int64_t kDtItems = 1024;  // four workgroups per CU
 
 // Host-side launch context: kernel constants plus the launch ranges.
 struct LaunchCtx {
   KCtx k;
   int limiter, riemann, metric, recovery;
+  int maxblocks = 1;               // largest number of blocks of one mesh
   Range3 interior, entire, face[3], ct;
   Range3 fixx1;  // the entire range in runs of 248 cells (k_fix_flux_x1)
   Range3 x1cells;                  // cell range of the shared-reconstruction X1 sweep

@@ -1022,44 +1022,59 @@ __global__ __launch_bounds__(256) void k_dt_reduce(KCtx C, double *const *alfven
 // Harmonic combination per block (timestep_estimation.cc:94-98), minimum
 // over the blocks of one mesh, then dt control dt_next = min(dt_factor * dt,
 // estimate) and time += dt.  One workgroup per mesh m: state + 2m = {dt,
-// time}; est_out (optional) + m gets the estimate.
-__global__ __launch_bounds__(256) void k_dt_final(KCtx C, const double *red, double *state,
-                                                  double dt_factor, double *est_out) {
-  __shared__ double sm[256];
+// time}; est_out (optional) + m gets the estimate.  W lanes share a block's
+// items, which the maximum lets them read in any order: the kernel is a few
+// memory round trips long, and one lane walking a block's items made it
+// longer with every item.
+template <int W>
+__global__ __launch_bounds__(1024) void k_dt_final(KCtx C, const double *red, double *state,
+                                                   double dt_factor, double *est_out) {
+  __shared__ double sm[16];
   const int m = blockIdx.x;
+  const int lane = (int)threadIdx.x & (W - 1), grp = (int)threadIdx.x / W;
   double mn = DBL_MAX;
-  for (int b = C.mfirst[m] + (int)threadIdx.x; b < C.mfirst[m + 1]; b += blockDim.x) {
+  for (int b = C.mfirst[m] + grp; b < C.mfirst[m + 1]; b += 1024 / W) {
     const DevBlock &B = C.blk[b];
+    const int p1 = C.dtfirst[b + 1];
+    double cmax[3] = {0.0, 0.0, 0.0};
+    for (int p = C.dtfirst[b] + lane; p < p1; p += 4 * W) {
+      double w[4][3];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) w[u][d] = (p + u * W < p1) ? red[(int64_t)(p + u * W) * 3 + d] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) cmax[d] = (w[u][d] > cmax[d]) ? w[u][d] : cmax[d];
+    }
+#pragma unroll
+    for (int off = W / 2; off > 0; off >>= 1)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const double o = __shfl_xor(cmax[d], off, W);
+        cmax[d] = (o > cmax[d]) ? o : cmax[d];
+      }
     double q3[3] = {DBL_MAX, DBL_MAX, DBL_MAX};
+#pragma unroll
     for (int d = 0; d < 3; ++d) {
       if (B.n[d] == 1) continue;
-      // the block's items, 16 independent loads at a time
-      double cmax = 0.0;
-      const int p1 = C.dtfirst[b + 1];
-      for (int p0 = C.dtfirst[b]; p0 < p1; p0 += 16) {
-        double w[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) w[u] = (p0 + u < p1) ? red[(int64_t)(p0 + u) * 3 + d] : 0.0;
-#pragma unroll
-        for (int u = 0; u < 16; ++u) cmax = (w[u] > cmax) ? w[u] : cmax;
-      }
-      const double q = C.ph.cfl * B.dx[d] / cmax;
+      const double q = C.ph.cfl * B.dx[d] / cmax[d];
       q3[d] = (q < DBL_MAX) ? q : DBL_MAX;
     }
     const double t = 1.0 / (1.0 / q3[0] + 1.0 / q3[1] + 1.0 / q3[2]);
     if (t < mn) mn = t;
   }
-  sm[threadIdx.x] = mn;
-  __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) {
-      const double o = sm[threadIdx.x + s];
-      if (o < sm[threadIdx.x]) sm[threadIdx.x] = o;
-    }
-    __syncthreads();
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const double o = __shfl_xor(mn, off, 64);
+    if (o < mn) mn = o;
   }
+  if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = mn;
+  __syncthreads();
   if (threadIdx.x == 0) {
-    const double est = sm[0];
+    double est = sm[0];
+    for (int q = 1; q < 16; ++q) est = (sm[q] < est) ? sm[q] : est;
     if (est_out) est_out[m] = est;
     if (state) {
       double *st = state + 2 * m;
@@ -1345,8 +1360,12 @@ int launch_dt(const LaunchCtx &L, double *const *alfven, double *red, double *st
   else
     hipLaunchKernelGGL(k_dt_reduce<16>, dim3(L.k.ndt), dim3(256), 0, s, L.k, alfven, red);
   TICK("dt_reduce");
-  hipLaunchKernelGGL(k_dt_final, dim3(L.k.nmesh), dim3(256), 0, s, L.k, red, state, dt_factor,
-                     est_out);
+  // a wavefront per block where no mesh has more than 16 blocks (a single
+  // block may hold hundreds of items), 16 lanes per block otherwise
+  if (L.maxblocks <= 16)
+    hipLaunchKernelGGL(k_dt_final<64>, dim3(L.k.nmesh), dim3(1024), 0, s, L.k, red, state, dt_factor, est_out);
+  else
+    hipLaunchKernelGGL(k_dt_final<16>, dim3(L.k.nmesh), dim3(1024), 0, s, L.k, red, state, dt_factor, est_out);
   TICK("dt_final");
   return PG_CHECK_LAUNCH();
 }

@@ -13,7 +13,7 @@ CASES = {
     "2d": [configs.orszag_tang(48, (2, 3, 1))],
     "3d_odd": [configs.torus3d((38, 22, 14), (2, 2, 2))],
     "3d_runs": [configs.torus3d((128, 96, 64), (2, 2, 1))],
-    "batch": [configs.torus2d(64, 32, (2, 2, 1)), configs.torus3d((32, 16, 16), (2, 1, 2)), configs.torus2d(40, 24)],
+    "batch": configs.ensemble(seed=3, n_tori=2, n_boxes_each=2, sizes3d=(16,), tori_res=((64, 32), (80, 48))),
 }
 
 
