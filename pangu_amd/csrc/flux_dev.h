@@ -78,7 +78,7 @@ __device__ __forceinline__ void face_flux(const KCtx &C, const KFields &F, doubl
   contravariant_flux<0, HB>(gam, pr, sr, sg, UR);
   contravariant_flux<DIR, HB>(gam, pl, sl, sg, FL);
   contravariant_flux<DIR, HB>(gam, pr, sr, sg, FR);
-  const double den = cmax + cmin + 1e-20, rden = 1.0 / den;
+  const double den = cmax + cmin + 1e-20, rden = quot(1.0, den);
 #pragma unroll
   for (int q = 0; q < NC; ++q) {
     const int s = slot_of<HB, HK>(q);

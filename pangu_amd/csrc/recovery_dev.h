@@ -373,25 +373,27 @@ __device__ int c2p_1d(const double U[9], double p[9], double gamma, const CenMet
 }
 
 // ----------------------------------------------------- Kastaun et al. 2021
-// scheme_kastaun.h:84-108.
+// scheme_kastaun.h:84-108.  The divisions and the root of an evaluation run
+// through quot and root (exact_div.h), the search's through quot: five
+// divisions and a square root are most of an evaluation.
 __device__ __forceinline__ double kastaun_root(double mu, double D, double q, double bsq, double rsq,
                                                double rbsq, double gamma) {
-  const double x = 1.0 / (1.0 + mu * bsq);
+  const double x = quot(1.0, 1.0 + mu * bsq);
   const double xsq = x * x;
   const double rbarsq = x * (rsq * x + mu * (x + 1.0) * rbsq);
   const double musq = mu * mu;
   double vsq = musq * rbarsq;
   vsq = kmin(kmax(vsq, 0.0), 1.0 - 1.0e-14);
-  const double il = sqrt(1.0 - vsq);
+  const double il = root(1.0 - vsq);
   const double qbar = q - 0.5 * bsq - 0.5 * musq * xsq * (bsq * rsq - rbsq);
   const double eod = qbar - mu * rbarsq + 1.0;
   const double rho = D * il;
   double eps = D * eod - rho;
   eps = kmax(eps, 1.0e-300);
   const double pr = (gamma - 1.0) * eps;
-  const double hh = 1.0 + (eps + pr) / rho;
-  const double nu = kmax(hh * il, eod + pr / D);
-  return mu - 1.0 / (nu + mu * rbarsq);
+  const double hh = 1.0 + quot(eps + pr, rho);
+  const double nu = kmax(hh * il, eod + quot(pr, D));
+  return mu - quot(1.0, nu + mu * rbarsq);
 }
 
 // Kastaun inputs (scheme_kastaun.h:167-213): D, q = tau/D, r^2, b^2, (r.b)^2
@@ -493,14 +495,14 @@ __device__ __forceinline__ int kastaun_iterate(const KastaunIn &k, double gamma,
   mu = lo;
   for (int it = 0; it < MAX_NEWT_ITER; ++it) {
     const double old = mu;
-    mu = (fhi * lo - flo * hi) / (fhi - flo);
+    mu = quot(fhi * lo - flo * hi, fhi - flo);
     const double fm = kastaun_root(mu, D, q, bsq, rsq, rbsq, gamma);
     iters = it + 1;
     if (!isfinite(mu) || !isfinite(fm)) return 3;
-    if (fabs((mu - old) / (mu + 1.0e-300)) <= NEWT_TOL) return 0;
+    if (fabs(quot(mu - old, mu + 1.0e-300)) <= NEWT_TOL) return 0;
     if (fm * flo >= 0.0) {
       if (side == 1) {
-        const double wgt = 1.0 - fm / flo;
+        const double wgt = 1.0 - quot(fm, flo);
         fhi = (wgt > 0.0) ? fhi * wgt : 0.5 * fhi;
       }
       lo = mu;
@@ -508,7 +510,7 @@ __device__ __forceinline__ int kastaun_iterate(const KastaunIn &k, double gamma,
       side = 1;
     } else {
       if (side == -1) {
-        const double wgt = 1.0 - fm / fhi;
+        const double wgt = 1.0 - quot(fm, fhi);
         flo = (wgt > 0.0) ? flo * wgt : 0.5 * flo;
       }
       hi = mu;
