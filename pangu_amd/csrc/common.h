@@ -52,6 +52,14 @@ __device__ __forceinline__ void st32(T *base, uint32_t i, T v) {
   *(__attribute__((address_space(1))) T *)((__attribute__((address_space(1))) char *)base +
                                            i * (uint32_t)sizeof(T)) = v;
 }
+// st32 for values that no kernel reads before much else has gone through the
+// caches: the line is not kept in L2.
+template <class T>
+__device__ __forceinline__ void stnt32(T *base, uint32_t i, T v) {
+  __builtin_nontemporal_store(
+      v, (__attribute__((address_space(1))) T *)((__attribute__((address_space(1))) char *)base +
+                                                 i * (uint32_t)sizeof(T)));
+}
 // An array read and written element-wise through ld32 / st32: a[i] reads
 // or assigns element i.
 template <class T>

@@ -277,7 +277,7 @@ __device__ __forceinline__ void div_update_cell(const KCtx &C, const KFields &F0
     }
   }
 #pragma unroll
-  for (int q = 0; q < NC; ++q) glb(F1.cons[b * NC + q])[id] = unew[q];
+  for (int q = 0; q < NC; ++q) stnt32(F1.cons[b * NC + q], (uint32_t)id, unew[q]);  // next read a stage later
   if (uout) {
 #pragma unroll
     for (int q = 0; q < NC; ++q) uout[q] = unew[q];
