@@ -99,7 +99,12 @@ __device__ __forceinline__ double vsq_of_w(double Bsq, double QdotBsq, double Qt
 }
 
 // ------------------------------------------------- 2D (W, v^2) Newton scheme
-// scheme_2d.h:99-404.
+// scheme_2d.h:99-404.  The step's divisions run through quot (exact_div.h),
+// the three by gamma sharing one reciprocal, except where a failing cell can
+// divide by zero and come back (t36, and v^2 in the error): eleven divisions
+// are most of a step, and the steps are one dependent chain (with the 1Dvsq
+// scheme's: 2-D torus 512x256, chainer, 182 -> 175 us per cycle,
+// Orszag-Tang 256^2, 1Dvsq, 79.7 -> 77.9 us).
 template <int MF = FORM_FULL>
 __device__ int c2p_2d(const double U[9], double p[9], double gamma, const CenMetric &m, int &iters) {
   iters = 0;
@@ -127,18 +132,18 @@ __device__ int c2p_2d(const double U[9], double p[9], double gamma, const CenMet
   while (keep) {
     const double W = x0, vsq = x1, Wsq = W * W;
     const double gtmp = 1. - vsq;
-    const double p_tmp = ((gamma - 1.) * (W * gtmp - D * sqrt(gtmp)) / gamma);
-    const double dPdW = ((gamma - 1.) * (1. - vsq) / gamma);
-    const double dPdvsq = ((gamma - 1.) * (0.5 * D / sqrt(1. - vsq) - W) / gamma);
+    const double p_tmp = quot((gamma - 1.) * (W * gtmp - D * sqrt(gtmp)), gamma);
+    const double dPdW = quot((gamma - 1.) * (1. - vsq), gamma);
+    const double dPdvsq = quot((gamma - 1.) * (quot(0.5 * D, sqrt(1. - vsq)) - W), gamma);
     const double t2 = -0.5 * Bsq + dPdvsq;
     const double t3 = Bsq + W;
     const double t4 = t3 * t3;
-    const double t9 = 1.0 / Wsq;
+    const double t9 = quot(1.0, Wsq);
     const double t11 = Qtsq - vsq * t4 + QdotBsq * (Bsq + 2.0 * W) * t9;
     const double t16 = QdotBsq * t9;
     const double t18 = -Qdotn - 0.5 * Bsq * (1.0 + vsq) + 0.5 * t16 - W + p_tmp;
-    const double t21 = 1.0 / t3;
-    const double t23 = 1.0 / W;
+    const double t21 = quot(1.0, t3);
+    const double t23 = quot(1.0, W);
     const double t24 = t16 * t23;
     const double t25 = -1.0 + dPdW - t24;
     const double t35 = t25 * t3 + (Bsq - 2.0 * dPdvsq) * (QdotBsq + vsq * Wsq * W) * t9 * t23;
@@ -151,7 +156,7 @@ __device__ int c2p_2d(const double U[9], double p[9], double gamma, const CenMet
     const double o0 = x0;
     x0 += dx0;
     x1 += dx1;
-    errx = (x0 == 0.) ? fabs(dx0) : fabs(dx0 / x0);
+    errx = (x0 == 0.) ? fabs(dx0) : fabs(quot(dx0, x0));
     errx += (x1 == 0.) ? fabs(dx1) : fabs(dx1 / x1);
     x0 = fabs(x0);
     x0 = (x0 > W_TOO_BIG) ? o0 : x0;
@@ -199,8 +204,8 @@ __device__ __forceinline__ double w_of_vsq(double D, double K, double vsq, doubl
   const double gtmp = (1. - vsq);
   rho = D * sqrt(gtmp);
   pr = (K * pow(rho, gamma));
-  uu = (pr / (gamma - 1.));
-  return ((rho + uu + pr) / gtmp);
+  uu = quot(pr, gamma - 1.);
+  return quot(rho + uu + pr, gtmp);
 }
 
 __device__ inline double vsq_residual(const double U[9], const CenMetric &m, double K, double gamma,
@@ -222,7 +227,8 @@ __device__ inline double vsq_residual(const double U[9], const CenMetric &m, dou
 // that makes it, and serve the next step and the final reconstruction: the
 // same arguments give the same bits, and each evaluation is a pow, which
 // bounds this scheme (n + 1 of them for n steps; evaluating afresh at the top
-// of every step and after the last takes 2 n + 1).
+// of every step and after the last takes 2 n + 1).  The divisions run through
+// quot (exact_div.h), as in the 2D scheme, but for the step itself.
 template <int MF = FORM_FULL>
 __device__ int c2p_1dvsq(const double U[9], double p[9], double gamma, const CenMetric &m,
                          int &iters, double x0 = -1.0) {
@@ -250,10 +256,10 @@ __device__ int c2p_1dvsq(const double U[9], double p[9], double gamma, const Cen
       const double Wsq = Wf * Wf;
       const double W3 = Wf * Wsq;
       const double dWdvsq =
-          ((gamma * (2. - gamma) * pr + (gamma - 1.) * rho) / (2. * (gamma - 1.) * (1. - vsq) * (1. - vsq)));
+          quot(gamma * (2. - gamma) * pr + (gamma - 1.) * rho, 2. * (gamma - 1.) * (1. - vsq) * (1. - vsq));
       const double fact = (Bsq + Wf);
-      const double resid = Qtsq - vsq * fact * fact + QdotBsq * (Bsq + 2. * Wf) / Wsq;
-      const double jac = -fact * (fact + 2. * dWdvsq * (vsq + QdotBsq / W3));
+      const double resid = Qtsq - vsq * fact * fact + quot(QdotBsq * (Bsq + 2. * Wf), Wsq);
+      const double jac = -fact * (fact + 2. * dWdvsq * (vsq + quot(QdotBsq, W3)));
       const double dx = -resid / jac;
       f = 0.5 * resid * resid;
       df = -2. * f;
@@ -265,7 +271,7 @@ __device__ int c2p_1dvsq(const double U[9], double p[9], double gamma, const Cen
       const double Wo = W;
       W = w_of_vsq(D, K, x, gamma, pr, rho, uu);
       Wf = W;
-      errx = (W == 0.) ? fabs(W - Wo) : fabs((W - Wo) / W);
+      errx = (W == 0.) ? fabs(W - Wo) : fabs(quot(W - Wo, W));
       errx += (x == 0.) ? fabs(x - xo) : fabs((x - xo) / x);
     }
     if ((fabs(errx) <= NEWT_TOL) && (doing_extra == 0) && (EXTRA_NEWT_ITER > 0)) doing_extra = 1;
