@@ -267,6 +267,17 @@ static int build_geometry(pangu_ctx *c, const pangu_block *blocks) {
     if (upload(c, &dcen, cen.data(), cen.size())) return PANGU_EDEVICE;
     c->geo_bufs.push_back(dcen);
     G.cen = dcen;
+    auto null_table = [&](int d, int ni, int nj, int nk) -> int {
+      if (cfg.metric != PANGU_METRIC_CKS) return 0;
+      std::vector<double> tab((size_t)ni * nj * nk * 4);
+      geom::fill_null_table(cfg, H, d, ni, nj, nk, has3d, tab.data());
+      double *dt = nullptr;
+      if (upload(c, &dt, tab.data(), tab.size())) return -1;
+      c->geo_bufs.push_back(dt);
+      G.nul[d] = dt;
+      return 0;
+    };
+    if (null_table(3, G.ni, G.nj, G.nk)) return PANGU_EDEVICE;
     const int nfd = has3d ? 3 : 2;
     const int bdim = H.n[2] > 1 ? 3 : (H.n[1] > 1 ? 2 : 1);
     for (int d = 0; d < 3; ++d) {
@@ -285,6 +296,7 @@ static int build_geometry(pangu_ctx *c, const pangu_block *blocks) {
       if (upload(c, &dt, tab.data(), tab.size())) return PANGU_EDEVICE;
       c->geo_bufs.push_back(dt);
       G.face[d] = dt;
+      if (null_table(d, G.fi[d], G.fj[d], fk)) return PANGU_EDEVICE;
     }
     D.geo = (int)geos.size();
     key2geo[key] = D.geo;

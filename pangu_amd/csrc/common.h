@@ -156,6 +156,9 @@ struct DevGeo {
   int64_t ncen;         // ni*nj*nk
   int64_t nface[3];
   int fi[3], fj[3];     // face table row lengths (ni+1 / nj+1 on the normal dim)
+  // Cartesian Kerr-Schild: xi, l_1, l_2, l_3 of g = eta + xi l l at the faces
+  // of each direction and, [3], at the centres (laid out as the tables); else null
+  const double *nul[4];
   int conn_sym;         // every Gamma^a_{bc} equals Gamma^a_{cb} bit for bit: compact storage
   int pad;
 };

@@ -70,7 +70,7 @@ __device__ __forceinline__ void fix_cons_cell(const KCtx &C, const KFields &F, u
     const double u1 = p[UX1], u2 = p[UX2], u3 = p[UX3];
     const double *g = m.g;
     double uvsq = g[5] * u1 * u1 + g[10] * u2 * u2 + g[15] * u3 * u3;
-    if (MF == FORM_FULL) uvsq = uvsq + 2.0 * (g[6] * u1 * u2 + g[7] * u1 * u3 + g[11] * u2 * u3);
+    if (g_dense<MF>()) uvsq = uvsq + 2.0 * (g[6] * u1 * u2 + g[7] * u1 * u3 + g[11] * u2 * u3);
     if (MF == FORM_POLOIDAL) uvsq = uvsq + 2.0 * (g[7] * u1 * u3);
     const double umax2 = P.lorentz_max * P.lorentz_max - 1.0;
     if (umax2 > 0.0 && uvsq > umax2) {
@@ -554,7 +554,7 @@ int launch_fix_cons(const LaunchCtx &L, const KFields &F, uint8_t *const *mask, 
   else if (mf == FORM_FLAT)                                                                           \
     hipLaunchKernelGGL((k_fix_cons<FORM_FLAT, FX, CS, HB_, HK_>), g, wg, 0, s, L.k, F, mask, R);      \
   else                                                                                                \
-    hipLaunchKernelGGL((k_fix_cons<FORM_FULL, FX, CS, HB_, HK_>), g, wg, 0, s, L.k, F, mask, R)
+    hipLaunchKernelGGL((k_fix_cons<FORM_NULLV, FX, CS, HB_, HK_>), g, wg, 0, s, L.k, F, mask, R)
 #define FC2(FX, CS)                                \
   if (hb && hk) { FC(FX, CS, true, true); }        \
   else if (hb) { FC(FX, CS, true, false); }        \
@@ -606,7 +606,7 @@ static void flux_dir(const LaunchCtx &L, const KFields &F, double *const *alfven
   else if (mf == FORM_FLAT)                                                                       \
     hipLaunchKernelGGL((k_flux<DIR, LIM, RS, HB_, HK_, FORM_FLAT>), g, wg, 0, s, L.k, F, alfven, R); \
   else                                                                                            \
-    hipLaunchKernelGGL((k_flux<DIR, LIM, RS, HB_, HK_, FORM_FULL>), g, wg, 0, s, L.k, F, alfven, R)
+    hipLaunchKernelGGL((k_flux<DIR, LIM, RS, HB_, HK_, FORM_NULLV>), g, wg, 0, s, L.k, F, alfven, R)
 #define FL2(LIM, RS)                         \
   if (hb && hk) { FL(LIM, RS, true, true); } \
   else if (hb) { FL(LIM, RS, true, false); } \

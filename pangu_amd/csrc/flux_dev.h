@@ -28,25 +28,21 @@ __device__ __forceinline__ void face_flux(const KCtx &C, const KFields &F, doubl
   constexpr int NC = ncomp<HB, HK>();
   const DevGeo &G = C.geo[B.geo];
   double g[16], gc0[4], gdd = 1.0, sg = 1.0, alpha;
-  if (MF != FORM_FULL && DIR == 3) {  // no form but FULL depends on x3: the centre table serves
+  // the centre table serves X3 faces wherever the metric does not depend on x3
+  if (DIR == 3 && MF != FORM_NULLV && (MF != FORM_FULL || !G.face[2])) {
     const uint32_t t = (uint32_t)cen_index(G, k, j, i);
     auto comp = [&](int n) { return ldc32(G.cen, (int64_t)n * (uint32_t)G.ncen, t); };
-    load_metric<MF, CG_GCON, CG_ALPHA>(comp, g, gc0, alpha);
+    load_metric<MF, CG_GCON, CG_ALPHA>(comp, comp, g, gc0, alpha);
     if (MF != FORM_FLAT) {
       gdd = comp(CG_GCON + 15);
       sg = comp(CG_SG);
     }
-  } else if (DIR == 3 && !G.face[2]) {
-    const uint32_t t = (uint32_t)cen_index(G, k, j, i);
-    auto comp = [&](int n) { return ldc32(G.cen, (int64_t)n * (uint32_t)G.ncen, t); };
-    load_metric<MF, CG_GCON, CG_ALPHA>(comp, g, gc0, alpha);
-    gdd = comp(CG_GCON + 15);
-    sg = comp(CG_SG);
   } else {
     const int d = DIR - 1;
     const uint32_t t = (uint32_t)(((G.has3d ? k : 0) * G.fj[d] + j) * G.fi[d] + i);
     auto comp = [&](int n) { return ldc32(G.face[d], (int64_t)n * (uint32_t)G.nface[d], t); };
-    load_metric<MF, FG_GCON0, FG_ALPHA>(comp, g, gc0, alpha);
+    auto nul = [&](int n) { return ldc32(G.nul[d], (int64_t)n * (uint32_t)G.nface[d], t); };
+    load_metric<MF, FG_GCON0, FG_ALPHA>(comp, nul, g, gc0, alpha);
     if (MF != FORM_FLAT) {
       gdd = comp(FG_GCONDD);
       sg = comp(FG_SG);

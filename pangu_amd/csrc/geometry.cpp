@@ -83,8 +83,8 @@ static void boyer_lindquist(const double x[4], M4 g, double h, double a) {
   g[3][3] = r2 * s2 * (1.0 + a2 / r2 + 2.0 * a2 * s2 / (r * r2 * mu));
 }
 
-// Cartesian Kerr-Schild g = eta + xi l l (CKS.h:22-69).
-static void cartesian_ks(const double x[4], M4 g, double a) {
+// xi and l of Cartesian Kerr-Schild, g = eta + xi l l (CKS.h:22-69).
+static void null_vector(const double x[4], double a, double &xi, double l[4]) {
   const double X = x[1], Y = x[2], Z = x[3];
   const double a2 = a * a;
   const double q = (X * X + Y * Y + Z * Z) - a2;
@@ -92,9 +92,17 @@ static void cartesian_ks(const double x[4], M4 g, double a) {
   const double rr = (r > 1.0e-15) ? r : 1.0e-15;
   const double r2 = rr * rr, r3 = r2 * rr, r4 = r2 * r2;
   const double den = r4 + a2 * Z * Z;
-  const double xi = (den > 0.0) ? (2.0 * r3 / den) : 0.0;
+  xi = (den > 0.0) ? (2.0 * r3 / den) : 0.0;
   const double dl = r2 + a2;
-  const double l[4] = {1.0, (rr * X + a * Y) / dl, (rr * Y - a * X) / dl, Z / rr};
+  l[0] = 1.0;
+  l[1] = (rr * X + a * Y) / dl;
+  l[2] = (rr * Y - a * X) / dl;
+  l[3] = Z / rr;
+}
+
+static void cartesian_ks(const double x[4], M4 g, double a) {
+  double xi, l[4];
+  null_vector(x, a, xi, l);
   zero(g);
   g[0][0] = -1.0;
   g[1][1] = 1.0;
@@ -322,6 +330,29 @@ void fill_face_table(const pangu_config &cfg, const HostBlock &H, int d, int fi,
         if (d == 1) x[2] = H.xf(1, j);
         if (d == 2) x[3] = H.xf(2, kk);
         fill_face(cfg, d, x, out + ((int64_t)kk * fj + j) * fi + i, n);
+      }
+}
+
+// xi, l_1, l_2, l_3 at the same places.  The kernels form gcov from them with
+// the operations of cartesian_ks; the code metric adds nothing to it, since
+// the Jacobian of the identity map is exactly the unit matrix.
+void fill_null_table(const pangu_config &cfg, const HostBlock &H, int d, int fi, int fj, int fk, bool has3d,
+                     double *out) {
+  const int64_t n = (int64_t)fi * fj * fk;
+  const double x3c = H.xc(2, H.s[2]);
+#pragma omp parallel for schedule(static) collapse(2)
+  for (int kk = 0; kk < fk; ++kk)
+    for (int j = 0; j < fj; ++j)
+      for (int i = 0; i < fi; ++i) {
+        double x[4] = {0.0, H.xc(0, i), H.xc(1, j), has3d ? H.xc(2, kk) : x3c};
+        if (d == 0) x[1] = H.xf(0, i);
+        if (d == 1) x[2] = H.xf(1, j);
+        if (d == 2) x[3] = H.xf(2, kk);
+        double xi, l[4];
+        null_vector(x, cfg.a, xi, l);
+        const int64_t e = ((int64_t)kk * fj + j) * fi + i;
+        out[e] = xi;
+        for (int q = 1; q < 4; ++q) out[q * n + e] = l[q];
       }
 }
 

@@ -55,6 +55,10 @@ void fill_centre_table(const pangu_config &cfg, const HostBlock &H, int ni, int 
                        bool has3d, double *out);
 void fill_face_table(const pangu_config &cfg, const HostBlock &H, int d, int fi, int fj, int fk,
                      bool has3d, double *out);
+// Cartesian Kerr-Schild: 4 components at the faces normal to d (0..2) or the
+// centres (3).
+void fill_null_table(const pangu_config &cfg, const HostBlock &H, int d, int fi, int fj, int fk, bool has3d,
+                     double *out);
 }  // namespace geom
 
 

@@ -163,9 +163,9 @@ int mlp_device(const pangu_mlp *m);
 // Target of the model: 0 Kastaun bracket, 1 1Dvsq start.
 int mlp_kind(const pangu_mlp *m);
 
-// The structure of metric's tables (physics_dev.h).
+// The form the plain kernels of a metric are compiled for (physics_dev.h).
 inline int metric_form(int metric) {
-  return metric == PANGU_METRIC_MINKOWSKI ? FORM_FLAT : metric == PANGU_METRIC_CKS ? FORM_FULL : FORM_POLOIDAL;
+  return metric == PANGU_METRIC_MINKOWSKI ? FORM_FLAT : metric == PANGU_METRIC_CKS ? FORM_NULLV : FORM_POLOIDAL;
 }
 
 // Attaches (or, with nullptr, detaches) a clock to a context's launches.

@@ -343,8 +343,9 @@ template <int MF>
 __device__ __forceinline__ void load_cen_metric(const DevGeo &G, int64_t t, CenMetric &m, double &sg,
                                                 double &alpha) {
   auto comp = [&](int n) { return ldc32(G.cen, (int64_t)n * G.ncen, (uint32_t)t); };
+  auto nul = [&](int n) { return ldc32(G.nul[3], (int64_t)n * G.ncen, (uint32_t)t); };
   double gc0[4];
-  load_metric<MF, CG_GCON, CG_ALPHA>(comp, m.gcov, gc0, alpha);
+  load_metric<MF, CG_GCON, CG_ALPHA>(comp, nul, m.gcov, gc0, alpha);
 #pragma unroll
   for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -1207,16 +1208,16 @@ int launch_div_update(const LaunchCtx &L, int mode, const KFields &F0, const KFi
     case 3:
       if (mf == FORM_POLOIDAL) {
         DU2(3, FORM_POLOIDAL)
-      } else if (mf == FORM_FULL) {
-        DU2(3, FORM_FULL)
+      } else if (mf == FORM_NULLV) {
+        DU2(3, FORM_NULLV)
       }
       break;
     case 5: DU2(4, FORM_FLAT) break;
     default:
       if (mf == FORM_POLOIDAL) {
         DU2(4, FORM_POLOIDAL)
-      } else if (mf == FORM_FULL) {
-        DU2(4, FORM_FULL)
+      } else if (mf == FORM_NULLV) {
+        DU2(4, FORM_NULLV)
       } else {
         DU2(4, FORM_FLAT)
       }
@@ -1278,7 +1279,7 @@ int launch_recover(const LaunchCtx &L, const KFields &F, const SharedTabs &S, in
   else if (mf == FORM_FLAT)                                                                           \
     hipLaunchKernelGGL((k_recover<FORM_FLAT, R_, HB_, HK_, HE_>), g, wg, 0, s, L.k, F, S, R);         \
   else                                                                                                \
-    hipLaunchKernelGGL((k_recover<FORM_FULL, R_, HB_, HK_, HE_>), g, wg, 0, s, L.k, F, S, R)
+    hipLaunchKernelGGL((k_recover<FORM_NULLV, R_, HB_, HK_, HE_>), g, wg, 0, s, L.k, F, S, R)
 #define RC2(R_, HE_)                          \
   if (hb && hk) { RC(R_, true, true, HE_); }  \
   else if (hb) { RC(R_, true, false, HE_); }  \
@@ -1353,7 +1354,7 @@ int launch_update_recover(const LaunchCtx &L, const KFields &F0, const KFields &
   else if (mf == FORM_FLAT)
     launch_ur_rec<FORM_FLAT>(a, g, wg, s, rec, hb, hk, h);
   else
-    launch_ur_rec<FORM_FULL>(a, g, wg, s, rec, hb, hk, h);
+    launch_ur_rec<FORM_NULLV>(a, g, wg, s, rec, hb, hk, h);
   TICK("update_recovery");
   return PG_CHECK_LAUNCH();
 }

@@ -37,7 +37,13 @@ __device__ __forceinline__ double kmin(double a, double b) { return (b < a) ? b 
 // only the entries the form leaves open, and drops the terms whose metric
 // factor is exactly zero: adding +-0 leaves a finite sum unchanged (a sum of
 // zeros may differ in sign), so results equal those of the full sums.
-//   FULL      every entry (Cartesian Kerr-Schild); g_{0i} = g_{i0} bit for bit
+//   FULL      every entry (any metric: the launch options' kernels);
+//             g_{0i} = g_{i0} bit for bit
+//   NULLV     eta + xi l l (Cartesian Kerr-Schild): xi and l are read, and
+//             gcov is formed from them as the table was, (xi l_m) l_n
+//             (the 3-D tables of a refined mesh exceed every cache: 11 loads
+//             per face for 20, 10 per centre for 19; 359 -> 313 us per cycle
+//             of the refined mesh without a field)
 //   POLOIDAL  x2 decouples (Kerr-Schild in MKS, Boyer-Lindquist): g_{m2} = 0
 //             for m != 2, g^{02} = 0, and g_{mn} = g_{nm} bit for bit
 //   FLAT      diag(-1, 1, 1, 1): nothing is read
@@ -49,22 +55,28 @@ __device__ __forceinline__ double kmin(double a, double b) { return (b < a) ? b 
 // a field (HB false below).  Per cycle: 3-D torus 256x128x128 4.36 -> 4.19 ms,
 // 2-D torus 512x256 247 -> 233 us, Orszag-Tang 256^2 134 -> 118 us, refined
 // Cartesian Kerr-Schild without a field 458 -> 423 us.
-enum MetricForm { FORM_FULL = 0, FORM_POLOIDAL = 1, FORM_FLAT = 2 };
+enum MetricForm { FORM_FULL = 0, FORM_POLOIDAL = 1, FORM_FLAT = 2, FORM_NULLV = 3 };
+
+// No entry fixed at zero?
+template <int MF>
+__host__ __device__ constexpr bool g_dense() {
+  return MF == FORM_FULL || MF == FORM_NULLV;
+}
 
 // Is g_{rc} possibly non-zero?
 template <int MF>
 __host__ __device__ constexpr bool g_open(int r, int c) {
-  return MF == FORM_FULL || r == c || (MF == FORM_POLOIDAL && r != 2 && c != 2);
+  return g_dense<MF>() || r == c || (MF == FORM_POLOIDAL && r != 2 && c != 2);
 }
 // Table slot (4 r + c) that holds g_{rc}: symmetric entries share one.
 template <int MF>
 __host__ __device__ constexpr int g_slot(int r, int c) {
-  return (r > c && (MF != FORM_FULL || c == 0)) ? 4 * c + r : 4 * r + c;
+  return (r > c && (!g_dense<MF>() || c == 0)) ? 4 * c + r : 4 * r + c;
 }
 // Is g^{0m} possibly non-zero?
 template <int MF>
 __host__ __device__ constexpr bool g0_open(int m) {
-  return m == 0 || MF == FORM_FULL || (MF == FORM_POLOIDAL && m != 2);
+  return m == 0 || g_dense<MF>() || (MF == FORM_POLOIDAL && m != 2);
 }
 
 // g_{rc} x^c over c = C0 .. 3, added in ascending c.

@@ -446,7 +446,7 @@ __device__ __forceinline__ int kastaun_setup(const double U[9], const CenMetric 
   const double tau = -Qdotn - D;
   if (!isfinite(tau)) return 3;
   const double S0 = U[UX1], S1 = U[UX2], S2 = U[UX3];
-  if (MF == FORM_FULL) {
+  if (g_dense<MF>()) {
     k.Su[0] = i0 * S0 + i1 * S1 + i2 * S2;
     k.Su[1] = i1 * S0 + i3 * S1 + i4 * S2;
     k.Su[2] = i2 * S0 + i4 * S1 + i5 * S2;

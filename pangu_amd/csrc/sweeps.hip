@@ -86,7 +86,7 @@ static void launch_form(const LaunchCtx &L, const KFields &F, double *const *alf
   else if (mf == FORM_FLAT)
     hipLaunchKernelGGL((k_sweeps<LIM, RS, HB, HK, FORM_FLAT>), g, wg, 0, s, L.k, F, alfven, S);
   else
-    hipLaunchKernelGGL((k_sweeps<LIM, RS, HB, HK, FORM_FULL>), g, wg, 0, s, L.k, F, alfven, S);
+    hipLaunchKernelGGL((k_sweeps<LIM, RS, HB, HK, FORM_NULLV>), g, wg, 0, s, L.k, F, alfven, S);
 }
 template <int LIM, int RS>
 static void launch_fields(const LaunchCtx &L, const KFields &F, double *const *alfven, const SweepSet &S,

@@ -16,7 +16,7 @@ def _tables(kind, n=400):
     d["metric"] = abi.METRIC[kind]
     rng = np.random.default_rng(7)
     dp = C.POINTER(C.c_double)
-    cen, face = [], []
+    cen, face, xs, spins = [], [], [], []
     for a, h in ((0.9375, 0.3), (0.0, 0.0), (-0.5, 0.9)):
         d.update(a=a, h=h)
         cfg = abi.config_from(d)
@@ -30,16 +30,23 @@ def _tables(kind, n=400):
             c = np.zeros(abi.CENTRE_NCOMP)
             assert L.pangu_geometry_entry(C.byref(cfg), 0, x.ctypes.data_as(dp), c.ctypes.data_as(dp)) == abi.OK
             cen.append(c)
+            xs.append(x)
+            spins.append(a)
             for dd in (1, 2, 3):
                 f = np.zeros(abi.FACE_NCOMP)
                 assert L.pangu_geometry_entry(C.byref(cfg), dd, x.ctypes.data_as(dp), f.ctypes.data_as(dp)) == abi.OK
                 face.append(f)
-    return np.array(cen), np.array(face)
+    return np.array(cen), np.array(face), xs, spins
+
+
+def _points(kind):
+    cen, _, xs, spins = _tables(kind)
+    return xs, spins, cen
 
 
 @pytest.mark.parametrize("kind", ["mks", "bl", "cks", "minkowski"])
 def test_tables_have_the_metric_form(kind):
-    cen, face = _tables(kind)
+    cen, face, _, _ = _tables(kind)
     for tab, g00 in ((cen, cen[:, 16:20]), (face, face[:, 16:20])):
         g = tab[:, :16].reshape(-1, 4, 4)
         # every form: the time row equals the time column
@@ -63,5 +70,19 @@ def test_tables_have_the_metric_form(kind):
         assert np.array_equal(cen[:, 16:32].reshape(-1, 4, 4), g[: len(cen)])
         assert np.all(cen[:, 32:35] == 1.0)
         assert np.all(face[:, 20:24] == 1.0)
+    if kind == "cks":
+        # eta + (xi l_m) l_n, from x as the tables' null vectors are
+        for x, a, c in zip(*_points(kind)):
+            X, Y, Z = x[1:]
+            a2 = a * a
+            q = (X * X + Y * Y + Z * Z) - a2
+            r = max(np.sqrt(0.5 * (q + np.sqrt(q * q + 4.0 * a2 * Z * Z))), 1.0e-15)
+            r2 = r * r
+            xi = 2.0 * (r2 * r) / (r2 * r2 + a2 * Z * Z)
+            l = [1.0, (r * X + a * Y) / (r2 + a2), (r * Y - a * X) / (r2 + a2), Z / r]
+            for m in range(4):
+                for n in range(4):
+                    eta = (-1.0 if m == 0 else 1.0) if m == n else 0.0
+                    assert c[4 * m + n] == eta + (xi * l[m]) * l[n]
     # a face is singular exactly where its lapse entry is zero
     assert np.array_equal(face[:, 22] == 0.0, face[:, 23] == 0.0)
