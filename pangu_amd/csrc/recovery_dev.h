@@ -153,7 +153,7 @@ __device__ int c2p_2d(const double U[9], double p[9], double gamma, const CenMet
     const double dx1 = -(-t25 * t11 - 2.0 * t40 * t18) * t21 * t36;
     df = -t11 * t11 - t18 * t18;
     f = -0.5 * df;
-    const double o0 = x0;
+    const double o0 = x0, o1 = x1;
     x0 += dx0;
     x1 += dx1;
     errx = (x0 == 0.) ? fabs(dx0) : fabs(quot(dx0, x0));
@@ -168,6 +168,16 @@ __device__ int c2p_2d(const double U[9], double p[9], double gamma, const CenMet
         (n_iter >= (MAX_NEWT_ITER - 1)))
       keep = false;
     n_iter++;
+    // A step that ends where it began without converging repeats itself to
+    // the last: cold cells at rest (v^2 below rounding) step to v^2 < 0 and
+    // are put back to 0 every time.  A tenth of a torus's cells do, in most
+    // of its wavefronts; their result and step count are those of the last
+    // step (update and recovery in the first cycles of the 2-D torus 512x256:
+    // 55.6 -> 34.3 us per launch).
+    if (doing_extra == 0 && x0 == o0 && x1 == o1) {
+      n_iter = MAX_NEWT_ITER;
+      keep = false;
+    }
   }
   iters = n_iter;
   int retval = 0;
