@@ -231,8 +231,8 @@ int pangu_get_tile_order(const pangu_ctx *ctx, int kernel_family);
 /* Cells per tile (threads per workgroup) of a kernel family's launches:
  * 256 (default), 128 or 64.  Smaller tiles waste fewer lanes on planes of
  * small blocks (a 10x10 face plane fills 100 of 256 lanes).  The flux
- * sweeps use it in their one-lane-per-face form only.  Results are
- * identical. */
+ * sweeps use it in their one-lane-per-face form only, and run in one launch
+ * only while all directions have the same size.  Results are identical. */
 int pangu_set_tile_size(pangu_ctx *ctx, int kernel_family, int cells);
 int pangu_get_tile_size(const pangu_ctx *ctx, int kernel_family);
 /* Fused stage only: split = 1 runs the geometric source in a kernel of its

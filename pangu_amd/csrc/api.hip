@@ -5,6 +5,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -19,6 +20,7 @@ using namespace pangu;
 struct DevContainer {
   std::vector<double *> hprim, hcons, hflux[3];
   double **dprim = nullptr, **dcons = nullptr, **dflux[3] = {nullptr, nullptr, nullptr};
+  int prim_of = 0;  // the first container registered that shares a primitive array with this one
   KFields kf() const {
     KFields f;
     f.prim = dprim;
@@ -960,6 +962,14 @@ int pangu_register_container(pangu_ctx *c, const pangu_container *src, int *hand
     }
   }
   *handle = (int)c->conts.size();
+  d.prim_of = *handle;
+  const std::set<double *> mine(d.hprim.begin(), d.hprim.end());
+  for (int h = *handle - 1; h >= 0; --h)
+    for (double *q : c->conts[h].hprim)
+      if (mine.count(q)) {
+        d.prim_of = c->conts[h].prim_of;
+        break;
+      }
   c->conts.push_back(d);
   return PANGU_OK;
 }
@@ -1178,7 +1188,9 @@ int pangu_stage(pangu_ctx *c, int md_init, int md0, int md1, double beta, double
   // default only on a refined mesh: elsewhere the cross-stream join costs
   // more than the overlap hides.
   const bool want = c->L.overlap_exchange > 0 || (c->L.overlap_exchange < 0 && c->L.ml.on);
-  const bool overlap = exchange_after == 0 && md1 != md0 && want && c->side && !c->L.clock;
+  // (Two handles on one set of primitives are one container here.)
+  const bool distinct = c->conts[md1].prim_of != c->conts[md0].prim_of;
+  const bool overlap = exchange_after == 0 && distinct && want && c->side && !c->L.clock;
   if (overlap) {
     HIPCHK(c, hipEventRecord(c->ev_fork, s));
     HIPCHK(c, hipStreamWaitEvent(c->side, c->ev_fork, 0));
@@ -1190,7 +1202,7 @@ int pangu_stage(pangu_ctx *c, int md_init, int md0, int md1, double beta, double
   const bool fuse_fx = c->L.fuse_fix_x1 && !c->L.share_x1 && !(c->L.pair_flux & 1);
   // For the same reason the exchange may share the sweeps' launch, which
   // saves its own and hides its memory traffic behind their arithmetic.
-  const bool ride = exchange_after == 0 && md1 != md0 && !overlap && !fuse_fx && exchange_rides(c->L);
+  const bool ride = exchange_after == 0 && distinct && !overlap && !fuse_fx && exchange_rides(c->L);
   if (fuse_fx) {
     LCHK(c, launch_fix_flux_x1(c->L, f0, c->dmask, c->dalfven, s));
     LCHK(c, launch_fluxes_23(c->L, f0, c->dalfven, s));
