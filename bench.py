@@ -72,12 +72,12 @@ LEARNED_GATES = (0, 5, 7)
 # (div_update_source and recovery_heating: the two kernels update_recovery
 # fuses, as they measured when they ran separately.)
 MEASURED = {
-    "update_recovery": {"bytes": 2618017375, "fp64_flops": 9.184e9},
+    "update_recovery": {"bytes": 2587516496, "fp64_flops": 8.452e9},
     "div_update_source": {"bytes": 2222250845, "fp64_flops": 2.634e9},
-    "flux_x1": {"bytes": 882992578, "fp64_flops": 5.640e9},
-    "flux_x2": {"bytes": 935706711, "fp64_flops": 5.584e9},
-    "flux_x3": {"bytes": 857050699, "fp64_flops": 5.098e9},
-    "fix_cons": {"bytes": 1120776037, "fp64_flops": 4.792e9},
+    "flux_x1": {"bytes": 888205342, "fp64_flops": 5.071e9},
+    "flux_x2": {"bytes": 934476128, "fp64_flops": 4.977e9},
+    "flux_x3": {"bytes": 848554676, "fp64_flops": 4.570e9},
+    "fix_cons": {"bytes": 1107508193, "fp64_flops": 4.269e9},
     "recovery_heating": {"bytes": 1034636023, "fp64_flops": 6.558e9},
 }
 
