@@ -125,6 +125,15 @@ static void physical(int kind, const double x[4], M4 g, double h, double a) {
 void code_metric(int kind, const double x[4], M4 out, double h, double a) {
   M4 g;
   physical(kind, x, g, h, a);
+  if (kind == PANGU_METRIC_CKS || kind == PANGU_METRIC_MINKOWSKI) {
+    // identity map: every J[c][c] is a number divided by itself and the rest
+    // are exactly 0, so the sums below come to 0 + g[r][c] (a centre entry of
+    // Cartesian Kerr-Schild, seven code metrics, took 5.9 us with them and
+    // takes 2.3 us)
+    for (int r = 0; r < 4; ++r)
+      for (int c = 0; c < 4; ++c) out[r][c] = 0.0 + g[r][c];
+    return;
+  }
   M4 J;
   zero(J);
   const double del = 1.0e-5;
