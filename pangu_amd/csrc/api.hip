@@ -20,7 +20,7 @@ using namespace pangu;
 struct DevContainer {
   std::vector<double *> hprim, hcons, hflux[3];
   double **dprim = nullptr, **dcons = nullptr, **dflux[3] = {nullptr, nullptr, nullptr};
-  int prim_of = 0;  // the first container registered that shares a primitive array with this one
+  std::set<int> sharing;  // earlier containers that have a primitive array in common with this one
   KFields kf() const {
     KFields f;
     f.prim = dprim;
@@ -962,12 +962,11 @@ int pangu_register_container(pangu_ctx *c, const pangu_container *src, int *hand
     }
   }
   *handle = (int)c->conts.size();
-  d.prim_of = *handle;
   const std::set<double *> mine(d.hprim.begin(), d.hprim.end());
-  for (int h = *handle - 1; h >= 0; --h)
+  for (int h = 0; h < *handle; ++h)
     for (double *q : c->conts[h].hprim)
       if (mine.count(q)) {
-        d.prim_of = c->conts[h].prim_of;
+        d.sharing.insert(h);
         break;
       }
   c->conts.push_back(d);
@@ -1041,6 +1040,12 @@ int pangu_calculate_conservative(pangu_ctx *c, int md, void *stream) {
 
 // Entry points that read or write face fluxes need the container's flux
 // tables on every active direction.
+// Do two handles have no primitive array in common?  (Sharing is a matter of
+// the pair: a third container may share some arrays with each of two that
+// share none.)
+static bool distinct_prims(const pangu_ctx *c, int a, int b) {
+  return a != b && !c->conts[std::max(a, b)].sharing.count(std::min(a, b));
+}
 static int need_fluxes(pangu_ctx *c, int md) {
   for (int d = 0; d < c->ndim; ++d)
     if (!c->conts[md].dflux[d]) return fail(c, PANGU_EINVAL, "container has no flux tables");
@@ -1182,14 +1187,14 @@ int pangu_stage(pangu_ctx *c, int md_init, int md0, int md1, double beta, double
   // container into its ghosts.  Nothing before the recovery writes that
   // interior P (the update writes U, FixPrimitive the input container's P)
   // or reads those ghosts or the flag, so with distinct input and output
-  // containers it runs on the side stream from the start of the stage,
-  // beside FixPrimitive and the flux sweeps, and joins before the recovery.
+  // containers (no primitive array in common) it runs on the side stream from
+  // the start of the stage, beside FixPrimitive and the flux sweeps, and
+  // joins before the recovery.
   // (Sequential when a kernel clock times the launches on one stream.)  By
   // default only on a refined mesh: elsewhere the cross-stream join costs
   // more than the overlap hides.
   const bool want = c->L.overlap_exchange > 0 || (c->L.overlap_exchange < 0 && c->L.ml.on);
-  // (Two handles on one set of primitives are one container here.)
-  const bool distinct = c->conts[md1].prim_of != c->conts[md0].prim_of;
+  const bool distinct = distinct_prims(c, md0, md1);
   const bool overlap = exchange_after == 0 && distinct && want && c->side && !c->L.clock;
   if (overlap) {
     HIPCHK(c, hipEventRecord(c->ev_fork, s));
