@@ -815,13 +815,11 @@ __device__ __forceinline__ void fix_cell(double *const *pp, int64_t id, int64_t 
   for (int q = 0; q < NP; ++q) glb(a[q])[id] = v[q];
 }
 
-// A failed cell that is not excised.
-__device__ __forceinline__ bool failed_cell(const KCtx &C, const DevBlock &B, const double *fl, int k, int j,
-                                            int i) {
-  if (glb(fl)[((int64_t)k * B.n[1] + j) * B.n[0] + i] != 0) return false;
-  if (C.ph.metric != PANGU_METRIC_CKS) return true;
+// Is cell (k, j, i) excised?
+__device__ __forceinline__ bool excised_cell(const KCtx &C, const DevBlock &B, int k, int j, int i) {
+  if (C.ph.metric != PANGU_METRIC_CKS) return false;
   const DevGeo &G = C.geo[B.geo];
-  return !(G.cen[CG_RAD * G.ncen + cen_index(G, k, j, i)] < C.ph.r_excise);
+  return G.cen[CG_RAD * G.ncen + cen_index(G, k, j, i)] < C.ph.r_excise;
 }
 
 template <int NP>
@@ -832,7 +830,7 @@ __global__ __launch_bounds__(256) void k_fixrec_a(KCtx C, KFields F, double *con
   const DevBlock &B = C.blk[b];
   const int64_t id = ((int64_t)k * B.n[1] + j) * B.n[0] + i;
   double *fl = flag[b];
-  if (!failed_cell(C, B, fl, k, j, i)) return;
+  if (fl[id] != 0 || excised_cell(C, B, k, j, i)) return;
   const int64_t jp = (B.s[1] != B.e[1]) ? (int64_t)B.n[0] : 0;
   const bool isolated = fl[id + jp - 1] != 0 && fl[id + jp] != 0 && fl[id + jp + 1] != 0 &&
                         fl[id + 1] != 0 && fl[id - jp + 1] != 0 && fl[id - jp] != 0 &&
@@ -846,17 +844,31 @@ __global__ __launch_bounds__(256) void k_fixrec_a(KCtx C, KFields F, double *con
 }
 
 // Phase B: one wavefront per interior (block, k) plane that holds clustered
-// cells (workgroup index = plane index).  Lane l walks row l of a band of 64
-// rows, two columns behind lane l - 1.  When a cell's turn comes, its
-// neighbours to the left and in the row before are done (the lane before is
-// past them) and those to the right and in the row after are untouched, as in
+// cells (workgroup index = plane index).  Lane r walks row r of a band of 64
+// rows, two columns behind lane r - 1: cell (r, c) is fixed in step c + 2 r.
+// When a cell's turn comes, its neighbours to the left and in the row before
+// are done and those to the right and in the row after are untouched, as in
 // the lexicographic order, and no lane reads what another writes in the same
-// step.  A band's steps span only the columns that hold failed cells.  The
-// first cycle of a 512x256 torus, whose atmosphere fails by the thousand, took
-// 90 ms when one lane fixed the plane's cells one by one, and takes 5.8 ms.
+// step.  The failed cells are looked up first, as one bit per row in a word
+// per step, and only steps with a bit set are taken (a cell's failure ends in
+// its own turn and no other): a step is two memory round trips long, and of a
+// band's ni + 126 steps a few clusters leave most empty.  The words of
+// kFixSteps steps are held at a time.
+// us per plane with        1 pair, 4 and 32 pairs of failed cells, all failed
+//   64x64   as it is          11     16     55      205
+//           every step taken  44     60     94      241
+//           cell by cell      32     47    186    11400
+//   512x256 as it is         237    242    285     4280
+//           every step taken 640    699   1058     5110
+//           cell by cell     686    701    833   375000
+// (cell by cell: one lane, rows in turn).  First cycle of a 512x256 torus,
+// whose atmosphere fails by the thousand: 5.0, 5.6 and 90 ms.
+constexpr int kFixSteps = 1024;
+
 template <int NP>
 __global__ __launch_bounds__(64) void k_fixrec_b(KCtx C, KFields F, double *const *flag,
                                                  int *cluster) {
+  __shared__ unsigned long long todo[kFixSteps];  // bit r: row r has a failed cell in this step
   const int b = C.pblock[blockIdx.x];
   const int kk = (int)blockIdx.x - C.pfirst[b];
   if (cluster[blockIdx.x] == 0) return;
@@ -867,41 +879,47 @@ __global__ __launch_bounds__(64) void k_fixrec_b(KCtx C, KFields F, double *cons
   const int lane = threadIdx.x;
   const int ni = B.e[0] - B.s[0] + 1;
   for (int j0 = B.s[1]; j0 <= B.e[1]; j0 += 64) {
-    const int rows = min(64, B.e[1] - j0 + 1), cells = rows * ni;
-    int lo = ni, hi = -1;  // columns of the band's failed cells
-    for (int t = lane; t < cells; t += 64 * 8) {
-      bool bad[8];
-      int col[8];
+    const int rows = min(64, B.e[1] - j0 + 1), steps = ni + 2 * (rows - 1);
+    const int64_t row0 = ((int64_t)k * B.n[1] + j0) * B.n[0] + B.s[0];
+    for (int s0 = 0; s0 < steps; s0 += kFixSteps) {
+      const int ns = min(kFixSteps, steps - s0);
+      for (int t = lane; t < ns; t += 64) todo[t] = 0ull;
+      __syncthreads();
+      // the columns that any row reaches in these steps
+      const int c0 = max(0, s0 - 2 * (rows - 1)), nc = min(ni, s0 + ns) - c0, cells = rows * nc;
+      for (int t = lane; t < cells; t += 64 * 8) {
+        double f[8];
+        int r[8], c[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int c = min(t + 64 * u, cells - 1), r = c / ni;
-        col[u] = c - r * ni;
-        bad[u] = failed_cell(C, B, fl, k, j0 + r, B.s[0] + col[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (bad[u]) {
-          lo = min(lo, col[u]);
-          hi = max(hi, col[u]);
+        for (int u = 0; u < 8; ++u) {
+          const int q = min(t + 64 * u, cells - 1);
+          r[u] = q / nc;
+          c[u] = c0 + q - r[u] * nc;
+          f[u] = glb(fl)[row0 + (int64_t)r[u] * B.n[0] + c[u]];
         }
-    }
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      lo = min(lo, __shfl_xor(lo, off, 64));
-      hi = max(hi, __shfl_xor(hi, off, 64));
-    }
-    const int steps = hi < lo ? 0 : hi - lo + 1 + 2 * (rows - 1);
-    for (int s = 0; s < steps; ++s) {
-      const int c = lo + s - 2 * lane;
-      if (lane < rows && c >= lo && c <= hi) {
-        const int i = B.s[0] + c, j = j0 + lane;
-        if (failed_cell(C, B, fl, k, j, i)) {
-          const int64_t id = ((int64_t)k * B.n[1] + j) * B.n[0] + i;
-          fix_cell<NP>(F.prim + b * NP, id, jp, fl);
-          fl[id] = 1;
+        for (int u = 0; u < 8; ++u) {
+          const int s = c[u] + 2 * r[u] - s0;
+          if (f[u] == 0 && s >= 0 && s < ns && !excised_cell(C, B, k, j0 + r[u], B.s[0] + c[u]))
+            atomicOr(&todo[s], 1ull << r[u]);
         }
       }
-      __threadfence_block();  // the next step of every lane sees this one's stores
+      __syncthreads();
+      for (int t = 0; t < ns; t += 64) {
+        const unsigned long long mine = t + lane < ns ? todo[t + lane] : 0ull;
+        uint64_t left = __ballot(mine != 0);
+        while (left) {
+          const int l = __ffsll((unsigned long long)left) - 1;
+          left &= left - 1;
+          if ((__shfl(mine, l, 64) >> lane) & 1) {
+            const int64_t id = row0 + (int64_t)lane * B.n[0] + (s0 + t + l - 2 * lane);
+            fix_cell<NP>(F.prim + b * NP, id, jp, fl);
+            fl[id] = 1;
+          }
+          __threadfence_block();  // the next step of every lane sees this one's stores
+        }
+      }
+      __syncthreads();
     }
   }
   if (lane == 0) cluster[blockIdx.x] = 0;
