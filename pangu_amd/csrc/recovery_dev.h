@@ -101,7 +101,7 @@ __device__ __forceinline__ double vsq_of_w(double Bsq, double QdotBsq, double Qt
 // ------------------------------------------------- 2D (W, v^2) Newton scheme
 // scheme_2d.h:99-404.  The step's divisions run through quot (exact_div.h),
 // the three by gamma sharing one reciprocal, except where a failing cell can
-// divide by zero and come back (t36, and v^2 in the error): eleven divisions
+// divide by zero and come back (t36, dP/dv^2, v^2 in the error): eleven divisions
 // are most of a step, and the steps are one dependent chain (with the 1Dvsq
 // scheme's: 2-D torus 512x256, chainer, 182 -> 175 us per cycle,
 // Orszag-Tang 256^2, 1Dvsq, 79.7 -> 77.9 us).
@@ -134,7 +134,11 @@ __device__ int c2p_2d(const double U[9], double p[9], double gamma, const CenMet
     const double gtmp = 1. - vsq;
     const double p_tmp = quot((gamma - 1.) * (W * gtmp - D * sqrt(gtmp)), gamma);
     const double dPdW = quot((gamma - 1.) * (1. - vsq), gamma);
-    const double dPdvsq = quot((gamma - 1.) * (quot(0.5 * D, sqrt(1. - vsq)) - W), gamma);
+    // at v^2 = 1 the division by sqrt(1 - v^2) is infinite, not quot's NaN: dx1
+    // comes to zero then, v^2 stays 1, and a last step that starts there
+    // ends in status 4
+    const double dPdvsq =
+        gtmp == 0. ? D * HUGE_VAL : quot((gamma - 1.) * (quot(0.5 * D, sqrt(1. - vsq)) - W), gamma);
     const double t2 = -0.5 * Bsq + dPdvsq;
     const double t3 = Bsq + W;
     const double t4 = t3 * t3;
