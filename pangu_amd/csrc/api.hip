@@ -641,6 +641,14 @@ namespace pangu {
 void set_kernel_clock(pangu_ctx *c, KernelClock *clock) {
   if (c) c->L.clock = clock;
 }
+std::string launch_options(const pangu_ctx *c) {
+  const LaunchCtx &L = c->L;
+  char t[160];
+  snprintf(t, sizeof(t), "ov%d ur%d ct%d fx%d ml%d:%d,%d,%d mlp%d:%d root%d flag%d", L.overlap_exchange,
+           L.fuse_update_recovery, L.fuse_ct, L.fuse_fix_x1, L.ml.on, L.ml.nfill, L.ml.nprol, L.ml.nflux,
+           c->mlp ? 1 + mlp_kind(c->mlp) : 0, c->mlp ? c->guess_gate : 0, c->droot ? 1 : 0, c->dflag ? 1 : 0);
+  return t;
+}
 }  // namespace pangu
 
 extern "C" {

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <string>
 #include <vector>
 
 #include "../../include/pangu_mlp.h"
@@ -170,6 +171,9 @@ inline int metric_form(int metric) {
 
 // Attaches (or, with nullptr, detaches) a clock to a context's launches.
 void set_kernel_clock(pangu_ctx *c, KernelClock *clock);
+// What selects a fused stage's launches beside the blocks' shapes, the
+// physics and the options the autotuner sets, as text (part of its cache key).
+std::string launch_options(const pangu_ctx *c);
 
 int launch_fix_cons(const LaunchCtx &L, const KFields &F, uint8_t *const *mask, bool fix, bool cons,
                     hipStream_t s);

@@ -749,24 +749,40 @@ struct Tuning {
 };
 static std::map<std::string, Tuning> g_tune_cache;
 
-// Identifies a launch workload: block shapes and kernel-selecting options.
+// Identifies a launch workload: the blocks' shapes and physical faces, and
+// everything but the tuned options that selects a cycle's launches (whole
+// cycles decide part of the choice: whether the exchange can join the sweeps,
+// what the update and the recovery share a launch with).
 static std::string tune_signature(const pangu_sim *s) {
   std::string k;
-  char buf[96];
+  char buf[128];
   const pangu_sim_cfg &c = s->cfg;
-  snprintf(buf, sizeof(buf), "m%d r%d l%d c%d B%d H%d g%d|", c.metric, c.riemann, c.limiter,
-           c.recovery, c.enable_B, c.enable_heating, c.ng);
+  snprintf(buf, sizeof(buf), "m%d r%d l%d c%d B%d H%d g%d x%d n%d|", c.metric, c.riemann, c.limiter,
+           c.recovery, c.enable_B, c.enable_heating, c.ng, c.exchange_after, s->nmesh);
   k += buf;
+  k += launch_options(s->ctx) + "|";
+  auto block = [&](int b) -> std::string {
+    const HostBlock &H = s->hb[b];
+    const pangu_sim_cfg &m = s->mcfg[s->bmesh[b]];
+    char t[64];
+    int faces = 0;
+    for (int d = 0; d < 3; ++d) {
+      const bool lo = H.lx[d] == 0, hi = (int64_t)H.lx[d] == ((int64_t)m.nb[d] << H.level) - 1;
+      faces = 4 * faces + (H.n[d] > 1 && lo && m.bc[d][0] != PANGU_BC_PERIODIC ? 1 : 0) +
+              (H.n[d] > 1 && hi && m.bc[d][1] != PANGU_BC_PERIODIC ? 2 : 0);
+    }
+    snprintf(t, sizeof(t), "%dx%dx%d@%d:%d", H.n[0], H.n[1], H.n[2], H.level, faces);
+    return t;
+  };
+  std::string last;
   int run = 0;
   for (int b = 0; b <= s->nblk; ++b) {
-    const bool same = b < s->nblk && b > 0 && s->hb[b].n[0] == s->hb[b - 1].n[0] &&
-                      s->hb[b].n[1] == s->hb[b - 1].n[1] && s->hb[b].n[2] == s->hb[b - 1].n[2];
-    if (b > 0 && !same) {
-      const HostBlock &H = s->hb[b - 1];
-      snprintf(buf, sizeof(buf), "%dx%dx%d*%d,", H.n[0], H.n[1], H.n[2], run);
-      k += buf;
+    const std::string now = b < s->nblk ? block(b) : std::string();
+    if (b > 0 && now != last) {
+      k += last + "*" + std::to_string(run) + ",";
       run = 0;
     }
+    last = now;
     ++run;
   }
   return k;

@@ -89,6 +89,43 @@ def test_autotune_restores_state_and_keeps_results():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("other", ["exchange_after", "outflow", "overlap", "separate_update", "refined"])
+def test_tuning_of_another_setting_is_not_reused(other):
+    """A choice found for one setting serves the same setting, without
+    running a cycle, and no other that changes a cycle's launches: a choice
+    that is reused takes no time."""
+    import time
+
+    from pangu_amd.sim import HipSim
+    cfg = configs.orszag_tang(40, (2, 2, 1))
+    alt = dict(cfg)
+    if other == "exchange_after":
+        alt["exchange_after"] = 1
+    if other == "outflow":
+        alt["bc"] = [[configs.OUTFLOW, configs.OUTFLOW]] + [list(p) for p in cfg["bc"][1:]]
+    if other == "refined":
+        alt["refine"] = [(1, (0.25, 0.25, -0.5), (0.5, 0.5, 0.5))]
+
+    def tune(c):
+        h = HipSim(c)
+        h.init()
+        if c is alt and other == "overlap":
+            h.set_overlap_exchange(1)
+        if c is alt and other == "separate_update":
+            h.set_fuse_update_recovery(0)
+        t0 = time.perf_counter()
+        h.autotune(cycles=4)
+        t = time.perf_counter() - t0
+        h.close()
+        return t
+
+    first = tune(cfg)  # measures, or finds what an earlier case measured
+    again = min(tune(cfg) for _ in range(3))
+    new, known = tune(alt), min(tune(alt) for _ in range(3))
+    assert again < 0.2 * new and known < 0.2 * new, (first, again, new, known)
+
+
+@pytest.mark.gpu
 def test_plain_loop_equals_batch():
     from pangu_amd.sim import HipSim, plain_loop
     ens = _small_ensemble()
