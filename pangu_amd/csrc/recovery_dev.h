@@ -473,10 +473,18 @@ __device__ __forceinline__ int kastaun_setup(const double U[9], const CenMetric 
   k.B[0] = B0;
   k.B[1] = B1;
   k.B[2] = B2;
-  const double Bu[4] = {0.0, B0, B1, B2};
-  const double Bd0 = lower<MF, 1>(m.gcov, 1, Bu);
-  const double Bd1 = lower<MF, 1>(m.gcov, 2, Bu);
-  const double Bd2 = lower<MF, 1>(m.gcov, 3, Bu);
+  // the six entries on and above the diagonal, as for det: the ones below may
+  // differ from them in the last place (Cartesian Kerr-Schild)
+  double Bd0 = B0, Bd1 = B1, Bd2 = B2;
+  if (g_dense<MF>()) {
+    Bd0 = g0 * B0 + g1 * B1 + g2 * B2;
+    Bd1 = g1 * B0 + g3 * B1 + g4 * B2;
+    Bd2 = g2 * B0 + g4 * B1 + g5 * B2;
+  } else if (MF == FORM_POLOIDAL) {
+    Bd0 = g0 * B0 + g2 * B2;
+    Bd1 = g3 * B1;
+    Bd2 = g2 * B0 + g5 * B2;
+  }
   const double Bsq = B0 * Bd0 + B1 * Bd1 + B2 * Bd2;
   const double Ssq = k.Su[0] * S0 + k.Su[1] * S1 + k.Su[2] * S2;
   const double SdotB = B0 * S0 + B1 * S1 + B2 * S2;
