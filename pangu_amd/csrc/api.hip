@@ -265,21 +265,19 @@ static int build_geometry(pangu_ctx *c, const pangu_block *blocks) {
                         sizeof(double) * (size_t)G.ncen);
       std::memcpy(&cen[(size_t)(CG_CONN * G.ncen)], compact.data(), compact.size() * sizeof(double));
     }
-    double *dcen = nullptr;
-    if (upload(c, &dcen, cen.data(), cen.size())) return PANGU_EDEVICE;
-    c->geo_bufs.push_back(dcen);
-    G.cen = dcen;
-    auto null_table = [&](int d, int ni, int nj, int nk) -> int {
-      if (cfg.metric != PANGU_METRIC_CKS) return 0;
-      std::vector<double> tab((size_t)ni * nj * nk * 4);
-      geom::fill_null_table(cfg, H, d, ni, nj, nk, has3d, tab.data());
+    // Cartesian Kerr-Schild: xi and l instead of gcov; the rows before them
+    // stay on the host
+    G.nullv = cfg.metric == PANGU_METRIC_CKS;
+    const int skip = G.nullv ? CG_NUL : 0;
+    if (G.nullv) geom::fill_null_table(cfg, H, 3, G.ni, G.nj, G.nk, has3d, &cen[(size_t)(CG_NUL * G.ncen)]);
+    auto table = [&](const std::vector<double> &tab, int64_t n, const double **row0) -> int {
       double *dt = nullptr;
-      if (upload(c, &dt, tab.data(), tab.size())) return -1;
+      if (upload(c, &dt, tab.data() + skip * n, tab.size() - (size_t)(skip * n))) return -1;
       c->geo_bufs.push_back(dt);
-      G.nul[d] = dt;
+      *row0 = (const double *)((uintptr_t)dt - (uintptr_t)(skip * n) * sizeof(double));
       return 0;
     };
-    if (null_table(3, G.ni, G.nj, G.nk)) return PANGU_EDEVICE;
+    if (table(cen, G.ncen, &G.cen)) return PANGU_EDEVICE;
     const int nfd = has3d ? 3 : 2;
     const int bdim = H.n[2] > 1 ? 3 : (H.n[1] > 1 ? 2 : 1);
     for (int d = 0; d < 3; ++d) {
@@ -294,11 +292,9 @@ static int build_geometry(pangu_ctx *c, const pangu_block *blocks) {
       G.nface[d] = (int64_t)G.fi[d] * G.fj[d] * fk;
       std::vector<double> tab((size_t)(G.nface[d] * FG_NCOMP));
       geom::fill_face_table(cfg, H, d, G.fi[d], G.fj[d], fk, has3d, tab.data());
-      double *dt = nullptr;
-      if (upload(c, &dt, tab.data(), tab.size())) return PANGU_EDEVICE;
-      c->geo_bufs.push_back(dt);
-      G.face[d] = dt;
-      if (null_table(d, G.fi[d], G.fj[d], fk)) return PANGU_EDEVICE;
+      if (G.nullv)
+        geom::fill_null_table(cfg, H, d, G.fi[d], G.fj[d], fk, has3d, &tab[(size_t)(FG_NUL * G.nface[d])]);
+      if (table(tab, G.nface[d], &G.face[d])) return PANGU_EDEVICE;
     }
     D.geo = (int)geos.size();
     key2geo[key] = D.geo;

@@ -31,12 +31,41 @@ __device__ __forceinline__ int64_t cen_index(const DevGeo &G, int k, int j, int 
   return ((int64_t)(G.has3d ? k : 0) * G.nj + j) * G.ni + i;
 }
 
+static_assert(CG_GCOV == 0 && FG_GCOV == 0 && (int)CG_NUL == (int)FG_NUL, "both tables keep gcov alike");
+
+// gcov = eta + (xi l_r) l_c as the host forms it; comp(n) loads component n.
+template <class LD>
+__device__ __forceinline__ void gcov_from_null(LD comp, double g[16]) {
+  const double xi = comp(CG_NUL), l[4] = {1.0, comp(CG_NUL + 1), comp(CG_NUL + 2), comp(CG_NUL + 3)};
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const double t = r ? xi * l[r] : xi;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const double u = c ? t * l[c] : t;
+      g[4 * r + c] = r != c ? u : (r ? 1.0 : -1.0) + u;
+    }
+  }
+}
+
+// gcov of a table entry of any metric (nullv: DevGeo's), for readers that are
+// not compiled per form.
+template <class LD>
+__device__ __forceinline__ void load_gcov(LD comp, int nullv, double g[16]) {
+  if (nullv) {
+    gcov_from_null(comp, g);
+  } else {
+#pragma unroll
+    for (int n = 0; n < 16; ++n) g[n] = comp(n);
+  }
+}
+
 // gcov, g^{0m} and the lapse of a table entry, as far as form MF leaves them
 // open; the symmetric partner of a loaded entry shares its register.
 // comp(n) loads component n; GCON0 and ALPHA are the table's component
-// numbers of g^{00} and of 1/sqrt(-g^{00}); nul(n) loads xi (n = 0) or l_n.
-template <int MF, int GCON0, int ALPHA, class LD, class LN>
-__device__ __forceinline__ void load_metric(LD comp, LN nul, double g[16], double gc0[4], double &alpha) {
+// numbers of g^{00} and of 1/sqrt(-g^{00}).
+template <int MF, int GCON0, int ALPHA, class LD>
+__device__ __forceinline__ void load_metric(LD comp, double g[16], double gc0[4], double &alpha) {
   if (MF == FORM_FLAT) {
 #pragma unroll
     for (int n = 0; n < 16; ++n) g[n] = (n % 5) ? 0.0 : (n ? 1.0 : -1.0);
@@ -46,24 +75,16 @@ __device__ __forceinline__ void load_metric(LD comp, LN nul, double g[16], doubl
     return;
   }
   if (MF == FORM_NULLV) {
-    const double xi = nul(0), l[4] = {1.0, nul(1), nul(2), nul(3)};
+    gcov_from_null(comp, g);
+  } else {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const double t = r ? xi * l[r] : xi;
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const double u = c ? t * l[c] : t;
-        g[4 * r + c] = r != c ? u : (r ? 1.0 : -1.0) + u;
+        const int slot = g_slot<MF>(r, c);
+        g[4 * r + c] = !g_open<MF>(r, c) ? 0.0 : (slot < 4 * r + c ? g[slot] : comp(slot));
       }
-    }
   }
-#pragma unroll
-  for (int r = 0; r < 4 && MF != FORM_NULLV; ++r)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int slot = g_slot<MF>(r, c);
-      g[4 * r + c] = !g_open<MF>(r, c) ? 0.0 : (slot < 4 * r + c ? g[slot] : comp(slot));
-    }
 #pragma unroll
   for (int n = 0; n < 4; ++n) gc0[n] = g0_open<MF>(n) ? comp(GCON0 + n) : 0.0;
   alpha = comp(ALPHA);
@@ -79,8 +100,7 @@ __device__ __forceinline__ void load_cen_state(const DevGeo &G, int64_t t, CenLo
   const int64_t s = G.ncen;
   const uint32_t t32 = (uint32_t)t;
   auto comp = [&](int n) { return ldc32(c, n * s, t32); };
-  auto nul = [&](int n) { return ldc32(G.nul[3], n * s, t32); };
-  load_metric<MF, CG_GCON, CG_ALPHA>(comp, nul, m.g, m.gc0, m.alpha);
+  load_metric<MF, CG_GCON, CG_ALPHA>(comp, m.g, m.gc0, m.alpha);
   m.sg = MF == FORM_FLAT ? 1.0 : comp(CG_SG);
 }
 

@@ -106,9 +106,14 @@ enum Slot { RHO = 0, ENY, UX1, UX2, UX3, BX1, BX2, BX3, ENT, KEL, NPRIM };
 // values a per-cell recomputation would produce.
 //
 // Cell-centre table (one entry per ghosted (j,i), or (k,j,i) for x3-dependent
-// metrics):
+// metrics).  Cartesian Kerr-Schild tables hold xi, l_1, l_2, l_3 of
+// g = eta + xi l l in the last four rows of gcov's place and none before them
+// (DevGeo::nullv; gcov_from_null gives gcov bit for bit): a table's pointer
+// leads to where row 0 would be.  With gcov as well the tables of a 3-D block
+// took 190 rows instead of 126.
 enum CentreComp {
   CG_GCOV = 0,          // 16: gcov[r][c] at CG_GCOV + 4r + c
+  CG_NUL = 12,          // 4: Cartesian Kerr-Schild, instead of gcov
   CG_GCON = 16,         // 16: gcon[r][c]
   CG_SG = 32,           // sqrt|det g|
   CG_ALPHA = 33,        // 1/sqrt(-gcon00)   (state lapse)
@@ -123,6 +128,7 @@ enum CentreComp {
 // Face table (lower faces normal to direction d):
 enum FaceComp {
   FG_GCOV = 0,    // 16
+  FG_NUL = 12,    // 4: Cartesian Kerr-Schild, instead of gcov
   FG_GCON0 = 16,  // 4: gcon[0][0..3]
   FG_GCONDD = 20, // gcon[d][d]
   FG_SG = 21,     // sqrt|det g|
@@ -156,11 +162,8 @@ struct DevGeo {
   int64_t ncen;         // ni*nj*nk
   int64_t nface[3];
   int fi[3], fj[3];     // face table row lengths (ni+1 / nj+1 on the normal dim)
-  // Cartesian Kerr-Schild: xi, l_1, l_2, l_3 of g = eta + xi l l at the faces
-  // of each direction and, [3], at the centres (laid out as the tables); else null
-  const double *nul[4];
   int conn_sym;         // every Gamma^a_{bc} equals Gamma^a_{cb} bit for bit: compact storage
-  int pad;
+  int nullv;            // Cartesian Kerr-Schild: rows CG_NUL and FG_NUL instead of gcov
 };
 
 // Index of the unordered pair (b, c) among (0,0) (0,1) (0,2) (0,3) (1,1) (1,2)

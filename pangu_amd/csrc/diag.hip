@@ -14,6 +14,7 @@
 
 #include <mutex>
 
+#include "cell_dev.h"
 #include "common.h"
 #include "kernels.h"
 #include "physics_dev.h"
@@ -89,8 +90,7 @@ __global__ __launch_bounds__(256) void k_diag(KCtx C, KFields F, const int *shel
       const auto c = glb(G.cen);
       const int64_t s = G.ncen;
       double g[16], gc0[4];
-#pragma unroll
-      for (int n = 0; n < 16; ++n) g[n] = c[(CG_GCOV + n) * s + t];
+      load_gcov([&](int n) { return c[n * s + t]; }, G.nullv, g);
 #pragma unroll
       for (int n = 0; n < 4; ++n) gc0[n] = c[(CG_GCON + n) * s + t];
       const double alpha = c[CG_ALPHA * s + t], sg = c[CG_SG * s + t];

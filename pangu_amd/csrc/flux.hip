@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256) void k_flux(KCtx C, KFields F, double *const *
 // (s..e+1, one transverse ghost layer) reconstructs its two states from
 // them: the stencil i-3..i+2 lies in the cell's row and in the window.  Same
 // operations and operands as the two kernels: identical results.
-template <int LIM, int RS, bool HB, bool HK>
+template <int LIM, int RS, bool HB, bool HK, int MF>
 __global__ __launch_bounds__(256) void k_fix_flux_x1(KCtx C, KFields F, uint8_t *const *mask,
                                                      double *const *alfven, Range3 R) {
   __shared__ double sp[NPRIM][256];
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256) void k_fix_flux_x1(KCtx C, KFields F, uint8_t 
   double p[NPRIM];
 #pragma unroll
   for (int q = 0; q < NPRIM; ++q) p[q] = 0.0;
-  if (valid) fix_cons_cell<FORM_FULL, true, true, HB, HK>(C, F, mask, b, k, j, i, own, p);
+  if (valid) fix_cons_cell<MF, true, true, HB, HK>(C, F, mask, b, k, j, i, own, p);
 #pragma unroll
   for (int q = 0; q < NPRIM; ++q) sp[q][x] = p[q];
   __syncthreads();
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256) void k_fix_flux_x1(KCtx C, KFields F, uint8_t 
       recon_mc(v[1], v[2], v[3], t1, pr[sl]);
     }
   }
-  face_flux<1, RS, HB, HK>(C, F, alfven, b, k, j, i, pl, pr);
+  face_flux<1, RS, HB, HK, MF>(C, F, alfven, b, k, j, i, pl, pr);
 }
 
 // The value of lane l - 1 (lane 0 gets 0) through the DPP wavefront shift
@@ -266,7 +266,7 @@ __device__ __forceinline__ double pair_swap(double x) {
 // order as k_flux, so the results are identical; what changes is that one
 // lane holds one fluid state instead of two (fewer registers, more
 // wavefronts in flight).
-template <int DIR, int LIM, int RS, bool HB, bool HK>
+template <int DIR, int LIM, int RS, bool HB, bool HK, int MF>
 __global__ __launch_bounds__(256) void k_flux_pair(KCtx C, KFields F, double *const *alfven, Range3 R) {
   int b = 0, k = 0, j = 0, i = 0;
   if (!decode_tile_pair(C, R, b, k, j, i)) return;  // both lanes of a pair share the outcome
@@ -324,8 +324,7 @@ __global__ __launch_bounds__(256) void k_flux_pair(KCtx C, KFields F, double *co
     const int64_t t = cen_index(G, k, j, i);
     const auto c = glb(G.cen);
     const int64_t ns = G.ncen;
-#pragma unroll
-    for (int n = 0; n < 16; ++n) g[n] = c[(CG_GCOV + n) * ns + t];
+    load_gcov([&](int n) { return c[n * ns + t]; }, MF == FORM_NULLV, g);
 #pragma unroll
     for (int n = 0; n < 4; ++n) gc0[n] = c[(CG_GCON + n) * ns + t];
     gdd = c[(CG_GCON + 15) * ns + t];
@@ -337,8 +336,7 @@ __global__ __launch_bounds__(256) void k_flux_pair(KCtx C, KFields F, double *co
     const int64_t t = ((int64_t)(G.has3d ? k : 0) * G.fj[d] + j) * G.fi[d] + i;
     const auto c = glb(G.face[d]);
     const int64_t ns = G.nface[d];
-#pragma unroll
-    for (int n = 0; n < 16; ++n) g[n] = c[(FG_GCOV + n) * ns + t];
+    load_gcov([&](int n) { return c[n * ns + t]; }, MF == FORM_NULLV, g);
 #pragma unroll
     for (int n = 0; n < 4; ++n) gc0[n] = c[(FG_GCON0 + n) * ns + t];
     gdd = c[FG_GCONDD * ns + t];
@@ -396,7 +394,7 @@ __global__ __launch_bounds__(256) void k_flux_pair(KCtx C, KFields F, double *co
 // Waves cover 64 consecutive cells of a plane's row-major cell range
 // (i = s - 1 .. e + 1) and overlap by one cell, so both neighbours of every
 // face sit in one wave.  Same arithmetic as k_flux<1>: identical results.
-template <int LIM, int RS, bool HB, bool HK>
+template <int LIM, int RS, bool HB, bool HK, int MF>
 __global__ __launch_bounds__(256) void k_flux_x1s(KCtx C, KFields F, double *const *alfven, Range3 R) {
   const int N = R.ntiles;
   const int n8 = (N + 7) >> 3;
@@ -449,7 +447,7 @@ __global__ __launch_bounds__(256) void k_flux_x1s(KCtx C, KFields F, double *con
     pl[s] = wave_shr1(rv[s]);
   }
   if (!have || lane == 0 || ic == 0) return;
-  face_flux<1, RS, HB, HK>(C, F, alfven, b, k, j, i, pl, pr);
+  face_flux<1, RS, HB, HK, MF>(C, F, alfven, b, k, j, i, pl, pr);
 }
 
 // Marching sweep along DIR (2 or 3): each thread walks R.step consecutive
@@ -464,7 +462,7 @@ __global__ __launch_bounds__(256) void k_flux_x1s(KCtx C, KFields F, double *con
 // instructions, and each face's loads wait for the previous face's physics
 // instead of overlapping other faces' work; the autotuner picks it only
 // where it wins.
-template <int DIR, int LIM, int RS, bool HB, bool HK>
+template <int DIR, int LIM, int RS, bool HB, bool HK, int MF>
 __global__ __launch_bounds__(256, 3) void k_flux_march(KCtx C, KFields F, double *const *alfven,
                                                     Range3 R) {
   int b = 0, k = 0, j = 0, i = 0, mend = 0;
@@ -529,7 +527,7 @@ __global__ __launch_bounds__(256, 3) void k_flux_march(KCtx C, KFields F, double
     // keep the carried states in LDS, not in registers, across the face
     // physics (the compiler would otherwise forward the stores)
     __asm__ volatile("" ::: "memory");
-    face_flux<DIR, RS, HB, HK>(C, F, alfven, b, k, j, i, pl, pr);
+    face_flux<DIR, RS, HB, HK, MF>(C, F, alfven, b, k, j, i, pl, pr);
     __asm__ volatile("" ::: "memory");
 #pragma unroll
     for (int q = 0; q < NC; ++q) {
@@ -593,14 +591,20 @@ static void flux_dir(const LaunchCtx &L, const KFields &F, double *const *alfven
   const dim3 g2((unsigned)(((2 * R.ntiles + 7) / 8) * 8));
   const bool hb = L.k.iBX >= 0, hk = L.k.iKEL >= 0;
   const int lim = L.limiter, rs = L.riemann, mf = metric_form(L.metric);
-#define FL(LIM, RS, HB_, HK_)                                                                      \
+#define FV(LIM, RS, HB_, HK_, MF_)                                                                 \
   if (shared)                                                                                     \
-    hipLaunchKernelGGL((k_flux_x1s<LIM, RS, HB_, HK_>), g, kTile, 0, s, L.k, F, alfven, R);       \
+    hipLaunchKernelGGL((k_flux_x1s<LIM, RS, HB_, HK_, MF_>), g, kTile, 0, s, L.k, F, alfven, R);  \
   else if (march)                                                                                 \
-    hipLaunchKernelGGL((k_flux_march<(DIR > 1 ? DIR : 2), LIM, RS, HB_, HK_>), g, kTile, 0, s, L.k, F, \
-                       alfven, R);                                                                \
-  else if (pair)                                                                                  \
-    hipLaunchKernelGGL((k_flux_pair<DIR, LIM, RS, HB_, HK_>), g2, kTile, 0, s, L.k, F, alfven, R); \
+    hipLaunchKernelGGL((k_flux_march<(DIR > 1 ? DIR : 2), LIM, RS, HB_, HK_, MF_>), g, kTile, 0, s, L.k, \
+                       F, alfven, R);                                                             \
+  else                                                                                            \
+    hipLaunchKernelGGL((k_flux_pair<DIR, LIM, RS, HB_, HK_, MF_>), g2, kTile, 0, s, L.k, F, alfven, R)
+#define FL(LIM, RS, HB_, HK_)                                                                      \
+  if ((shared || march || pair) && mf == FORM_NULLV) {                                            \
+    FV(LIM, RS, HB_, HK_, FORM_NULLV);                                                            \
+  } else if (shared || march || pair) {                                                           \
+    FV(LIM, RS, HB_, HK_, FORM_FULL);                                                             \
+  }                                                                                               \
   else if (mf == FORM_POLOIDAL)                                                                   \
     hipLaunchKernelGGL((k_flux<DIR, LIM, RS, HB_, HK_, FORM_POLOIDAL>), g, wg, 0, s, L.k, F, alfven, R); \
   else if (mf == FORM_FLAT)                                                                       \
@@ -623,6 +627,7 @@ static void flux_dir(const LaunchCtx &L, const KFields &F, double *const *alfven
   }
 #undef FL2
 #undef FL
+#undef FV
   TICK(DIR == 1 ? "flux_x1" : DIR == 2 ? "flux_x2" : "flux_x3");
 }
 
@@ -635,7 +640,12 @@ int launch_fluxes_23(const LaunchCtx &L, const KFields &F, double *const *alfven
 template <int LIM, int RS, bool HB, bool HK>
 static void launch_fx(const LaunchCtx &L, const Range3 &R, const KFields &F, uint8_t *const *mask,
                       double *const *alfven, hipStream_t s) {
-  hipLaunchKernelGGL((k_fix_flux_x1<LIM, RS, HB, HK>), tile_grid(R), kTile, 0, s, L.k, F, mask, alfven, R);
+  if (metric_form(L.metric) == FORM_NULLV)
+    hipLaunchKernelGGL((k_fix_flux_x1<LIM, RS, HB, HK, FORM_NULLV>), tile_grid(R), kTile, 0, s, L.k, F, mask,
+                       alfven, R);
+  else
+    hipLaunchKernelGGL((k_fix_flux_x1<LIM, RS, HB, HK, FORM_FULL>), tile_grid(R), kTile, 0, s, L.k, F, mask,
+                       alfven, R);
 }
 template <int LIM, int RS>
 static void launch_fx_fields(const LaunchCtx &L, const Range3 &R, const KFields &F, uint8_t *const *mask,

@@ -19,7 +19,7 @@ namespace pangu {
 // lower face of cell (k, j, i) along DIR: face metric, fluid states, fast
 // speeds, the four contravariant fluxes and the Riemann combine, from the
 // reconstructed left (pl) and right (pr) primitives.
-template <int DIR, int RS, bool HB, bool HK, int MF = FORM_FULL>
+template <int DIR, int RS, bool HB, bool HK, int MF>
 __device__ __forceinline__ void face_flux(const KCtx &C, const KFields &F, double *const *alfven, int b,
                                           int k, int j, int i, const double pl[NPRIM],
                                           const double pr[NPRIM]) {
@@ -32,7 +32,7 @@ __device__ __forceinline__ void face_flux(const KCtx &C, const KFields &F, doubl
   if (DIR == 3 && MF != FORM_NULLV && (MF != FORM_FULL || !G.face[2])) {
     const uint32_t t = (uint32_t)cen_index(G, k, j, i);
     auto comp = [&](int n) { return ldc32(G.cen, (int64_t)n * (uint32_t)G.ncen, t); };
-    load_metric<MF, CG_GCON, CG_ALPHA>(comp, comp, g, gc0, alpha);
+    load_metric<MF, CG_GCON, CG_ALPHA>(comp, g, gc0, alpha);
     if (MF != FORM_FLAT) {
       gdd = comp(CG_GCON + 15);
       sg = comp(CG_SG);
@@ -41,8 +41,7 @@ __device__ __forceinline__ void face_flux(const KCtx &C, const KFields &F, doubl
     const int d = DIR - 1;
     const uint32_t t = (uint32_t)(((G.has3d ? k : 0) * G.fj[d] + j) * G.fi[d] + i);
     auto comp = [&](int n) { return ldc32(G.face[d], (int64_t)n * (uint32_t)G.nface[d], t); };
-    auto nul = [&](int n) { return ldc32(G.nul[d], (int64_t)n * (uint32_t)G.nface[d], t); };
-    load_metric<MF, FG_GCON0, FG_ALPHA>(comp, nul, g, gc0, alpha);
+    load_metric<MF, FG_GCON0, FG_ALPHA>(comp, g, gc0, alpha);
     if (MF != FORM_FLAT) {
       gdd = comp(FG_GCONDD);
       sg = comp(FG_SG);

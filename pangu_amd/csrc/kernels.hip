@@ -343,9 +343,8 @@ template <int MF>
 __device__ __forceinline__ void load_cen_metric(const DevGeo &G, int64_t t, CenMetric &m, double &sg,
                                                 double &alpha) {
   auto comp = [&](int n) { return ldc32(G.cen, (int64_t)n * G.ncen, (uint32_t)t); };
-  auto nul = [&](int n) { return ldc32(G.nul[3], (int64_t)n * G.ncen, (uint32_t)t); };
   double gc0[4];
-  load_metric<MF, CG_GCON, CG_ALPHA>(comp, nul, m.gcov, gc0, alpha);
+  load_metric<MF, CG_GCON, CG_ALPHA>(comp, m.gcov, gc0, alpha);
 #pragma unroll
   for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -536,7 +535,7 @@ __global__ __launch_bounds__(256) void k_update_recover(KCtx C, KFields F0, KFie
 // the queue for the next launch on the stream, so a captured graph replays
 // it without a memset.  Tiles carry no dependencies, so no workgroup ever
 // waits for another.  Same cells, same arithmetic: identical results.
-template <int REC, bool HB, bool HK, bool HEAT>
+template <int MF, int REC, bool HB, bool HK, bool HEAT>
 __global__ __launch_bounds__(256) void k_recover_queue(KCtx C, KFields F, SharedTabs S, Range3 R,
                                                        unsigned *queue) {
   __shared__ int tile_sh;
@@ -547,7 +546,7 @@ __global__ __launch_bounds__(256) void k_recover_queue(KCtx C, KFields F, Shared
     __syncthreads();  // every thread has read the tile before the next pull
     if (T >= R.ntiles) break;
     int b, k, j, i;
-    if (decode_tile_at(C, R, T, b, k, j, i)) recover_cell<FORM_FULL, REC, HB, HK, HEAT>(C, F, S, b, k, j, i);
+    if (decode_tile_at(C, R, T, b, k, j, i)) recover_cell<MF, REC, HB, HK, HEAT>(C, F, S, b, k, j, i);
   }
   if (threadIdx.x == 0 && atomicAdd(&queue[1], 1u) == gridDim.x - 1) {
     atomicExch(&queue[0], 0u);
@@ -565,17 +564,19 @@ __global__ __launch_bounds__(256) void k_recover_queue(KCtx C, KFields F, Shared
 // k_recover; the recovered state agrees with it to the solver tolerance
 // (another false-position path to a root of the same function), not bit for
 // bit.
-template <bool HB, bool HK>
+template <int MF, bool HB, bool HK>
 __device__ __forceinline__ int learned_setup(const KCtx &C, const KFields &F, const DevGeo &G, int64_t t,
                                              int b, int64_t id, KastaunIn &kin) {
   constexpr int NC = ncomp<HB, HK>();
   const int64_t ns = G.ncen;
   CenMetric m;
+  auto comp = [&](int n) { return ldc32(G.cen, (int64_t)n * ns, (uint32_t)t); };
+  if (MF == FORM_NULLV)
+    gcov_from_null(comp, m.gcov);
+  else
+    load_gcov(comp, 0, m.gcov);
 #pragma unroll
-  for (int n = 0; n < 16; ++n) {
-    m.gcov[n] = ldc32(G.cen, (int64_t)(CG_GCOV + n) * ns, (uint32_t)t);
-    m.gcon[n] = ldc32(G.cen, (int64_t)(CG_GCON + n) * ns, (uint32_t)t);
-  }
+  for (int n = 0; n < 16; ++n) m.gcon[n] = comp(CG_GCON + n);
   m.lapse = ldc32(G.cen, (int64_t)CG_LAPSE * ns, (uint32_t)t);
   const double aos = ldc32(G.cen, (int64_t)CG_ALPHA * ns, (uint32_t)t) * (1.0 / ldc32(G.cen, (int64_t)CG_SG * ns, (uint32_t)t));
   const double *const *cons = F.cons + (int64_t)b * NC;
@@ -595,13 +596,13 @@ __device__ __forceinline__ int learned_setup(const KCtx &C, const KFields &F, co
 // UPD 1 or 2: the cell's update (k_div_update mode 4; 2 with the source)
 // runs first, as in k_update_recover; the recovery then reads the U this
 // thread has just stored.
-template <bool HB, bool HK, bool HEAT, int UPD>
+template <int MF, bool HB, bool HK, bool HEAT, int UPD>
 __global__ __launch_bounds__(256) void k_recover_learned(KCtx C, KFields F, SharedTabs S, MlpFrag W,
                                                          Range3 R, UpdArgs A) {
   int b = 0, k = 0, j = 0, i = 0;
   const bool cell = decode_tile(C, R, b, k, j, i);  // false on the whole workgroup past the range
   if (UPD && cell)
-    div_update_cell<4, UPD == 2 ? FORM_FULL : FORM_FLAT, HB, HK, HB>(C, A.F0, A.Finit, F, nullptr, A.dt_dev, A.beta, A.bdt_host, b,
+    div_update_cell<4, UPD == 2 ? MF : FORM_FLAT, HB, HK, HB>(C, A.F0, A.Finit, F, nullptr, A.dt_dev, A.beta, A.bdt_host, b,
                                              k, j, i, nullptr);
   const int lane = threadIdx.x & 63;
   constexpr int NC = ncomp<HB, HK>();
@@ -627,7 +628,7 @@ __global__ __launch_bounds__(256) void k_recover_learned(KCtx C, KFields F, Shar
   // every thread of the workgroup reaches the vote (no early return above)
   if (__syncthreads_or(gated)) {
     mlp_stage(W, lds, threadIdx.x, blockDim.x);
-    if (active) setup = learned_setup<HB, HK>(C, F, G, t, b, id, kin);
+    if (active) setup = learned_setup<MF, HB, HK>(C, F, G, t, b, id, kin);
     __syncthreads();
     const bool want = setup == 0;
     if (__ballot(gated && want)) {  // uniform over the wavefront: all 64 lanes run the network
@@ -643,10 +644,10 @@ __global__ __launch_bounds__(256) void k_recover_learned(KCtx C, KFields F, Shar
       // the setup is recomputed from memory (same inputs, same bits)
       // instead of being held in registers across the network
       __asm__ volatile("" ::: "memory");
-      if (active) setup = learned_setup<HB, HK>(C, F, G, t, b, id, kin);
+      if (active) setup = learned_setup<MF, HB, HK>(C, F, G, t, b, id, kin);
     }
   } else if (active) {
-    setup = learned_setup<HB, HK>(C, F, G, t, b, id, kin);
+    setup = learned_setup<MF, HB, HK>(C, F, G, t, b, id, kin);
   }
   if (!cell) return;
   Arr32<double> pp[NC];
@@ -710,11 +711,11 @@ __global__ __launch_bounds__(256) void k_recover_learned(KCtx C, KFields F, Shar
         for (int a = 0; a < 3; ++a) hp[BX1 + a] = bnew[a];
       }
       hp[ENT] = pp[ient<HB>()][id];
-      heat_vals<FORM_FULL, HB, HK>(C, F, G, t, b, id, pp, hp);
+      heat_vals<MF, HB, HK>(C, F, G, t, b, id, pp, hp);
       return;
     }
   }
-  if (HEAT && HK) heat_cell<FORM_FULL, HB, HK>(C, F, G, t, b, id, pp);
+  if (HEAT && HK) heat_cell<MF, HB, HK>(C, F, G, t, b, id, pp);
 }
 
 // The 1Dvsq recovery with the learned start (and, when HEAT, the heating):
@@ -725,13 +726,13 @@ __global__ __launch_bounds__(256) void k_recover_learned(KCtx C, KFields F, Shar
 // logistic(z) instead of the previous primitives' v^2.  Everything else is
 // recover_cell<2>: the result agrees with k_recover<2> to the Newton
 // tolerance, not bit for bit.
-template <bool HB, bool HK, bool HEAT, int UPD>
+template <int MF, bool HB, bool HK, bool HEAT, int UPD>
 __global__ __launch_bounds__(256) void k_recover_learned_vsq(KCtx C, KFields F, SharedTabs S, MlpFrag W,
                                                              Range3 R, UpdArgs A) {
   int b = 0, k = 0, j = 0, i = 0;
   const bool cell = decode_tile(C, R, b, k, j, i);  // false on the whole workgroup past the range
   if (UPD && cell)
-    div_update_cell<4, UPD == 2 ? FORM_FULL : FORM_FLAT, HB, HK, HB>(C, A.F0, A.Finit, F, nullptr, A.dt_dev, A.beta, A.bdt_host, b,
+    div_update_cell<4, UPD == 2 ? MF : FORM_FLAT, HB, HK, HB>(C, A.F0, A.Finit, F, nullptr, A.dt_dev, A.beta, A.bdt_host, b,
                                              k, j, i, nullptr);
   const int lane = threadIdx.x & 63;
   const Phys &P = C.ph;
@@ -750,7 +751,7 @@ __global__ __launch_bounds__(256) void k_recover_learned_vsq(KCtx C, KFields F, 
   if (__syncthreads_or(gated)) {
     mlp_stage(W, lds, threadIdx.x, blockDim.x);
     KastaunIn kin;
-    const int setup = active ? learned_setup<HB, HK>(C, F, G, t, b, id, kin) : -1;
+    const int setup = active ? learned_setup<MF, HB, HK>(C, F, G, t, b, id, kin) : -1;
     __syncthreads();
     const bool want = setup == 0;
     if (__ballot(gated && want)) {  // uniform over the wavefront: all 64 lanes run the network
@@ -766,7 +767,7 @@ __global__ __launch_bounds__(256) void k_recover_learned_vsq(KCtx C, KFields F, 
     }
   }
   if (!cell) return;
-  recover_cell<FORM_FULL, 2, HB, HK, HEAT>(C, F, S, b, k, j, i, x0);
+  recover_cell<MF, 2, HB, HK, HEAT>(C, F, S, b, k, j, i, x0);
 }
 
 // ---------------------------------------------------------- FixRecovery
@@ -1251,25 +1252,25 @@ int launch_div_update(const LaunchCtx &L, int mode, const KFields &F0, const KFi
   return PG_CHECK_LAUNCH();
 }
 
-template <bool HB, bool HK, bool HEAT>
+template <int MF, bool HB, bool HK, bool HEAT>
 static void launch_learned(const LaunchCtx &L, const KFields &F, const SharedTabs &S, const MlpFrag &W,
                            const Range3 &R, dim3 g, dim3 wg, hipStream_t s, const UpdArgs *upd) {
   const UpdArgs A = upd ? *upd : UpdArgs{};
   const int u = !upd ? 0 : (L.metric != PANGU_METRIC_MINKOWSKI ? 2 : 1);
   if (W.kind == 0) {
     if (u == 2)
-      hipLaunchKernelGGL((k_recover_learned<HB, HK, HEAT, 2>), g, wg, 0, s, L.k, F, S, W, R, A);
+      hipLaunchKernelGGL((k_recover_learned<MF, HB, HK, HEAT, 2>), g, wg, 0, s, L.k, F, S, W, R, A);
     else if (u == 1)
-      hipLaunchKernelGGL((k_recover_learned<HB, HK, HEAT, 1>), g, wg, 0, s, L.k, F, S, W, R, A);
+      hipLaunchKernelGGL((k_recover_learned<MF, HB, HK, HEAT, 1>), g, wg, 0, s, L.k, F, S, W, R, A);
     else
-      hipLaunchKernelGGL((k_recover_learned<HB, HK, HEAT, 0>), g, wg, 0, s, L.k, F, S, W, R, A);
+      hipLaunchKernelGGL((k_recover_learned<MF, HB, HK, HEAT, 0>), g, wg, 0, s, L.k, F, S, W, R, A);
   } else {
     if (u == 2)
-      hipLaunchKernelGGL((k_recover_learned_vsq<HB, HK, HEAT, 2>), g, wg, 0, s, L.k, F, S, W, R, A);
+      hipLaunchKernelGGL((k_recover_learned_vsq<MF, HB, HK, HEAT, 2>), g, wg, 0, s, L.k, F, S, W, R, A);
     else if (u == 1)
-      hipLaunchKernelGGL((k_recover_learned_vsq<HB, HK, HEAT, 1>), g, wg, 0, s, L.k, F, S, W, R, A);
+      hipLaunchKernelGGL((k_recover_learned_vsq<MF, HB, HK, HEAT, 1>), g, wg, 0, s, L.k, F, S, W, R, A);
     else
-      hipLaunchKernelGGL((k_recover_learned_vsq<HB, HK, HEAT, 0>), g, wg, 0, s, L.k, F, S, W, R, A);
+      hipLaunchKernelGGL((k_recover_learned_vsq<MF, HB, HK, HEAT, 0>), g, wg, 0, s, L.k, F, S, W, R, A);
   }
 }
 
@@ -1285,13 +1286,20 @@ int launch_recover(const LaunchCtx &L, const KFields &F, const SharedTabs &S, in
   const bool hb = L.k.iBX >= 0, hk = L.k.iKEL >= 0;
   const bool persist = L.persist_recovery && L.queue;
   const int mf = metric_form(L.metric);
+#define RQ(MF_, R_, HB_, HK_, HE_)                                                                    \
+  hipLaunchKernelGGL((k_recover_queue<MF_, R_, HB_, HK_, HE_>),                                       \
+                     dim3(resident_groups(k_recover_queue<MF_, R_, HB_, HK_, HE_>, R.tile, R.ntiles)), \
+                     wg, 0, s, L.k, F, S, R, L.queue)
 #define RC(R_, HB_, HK_, HE_)                                                                        \
-  if ((R_ == 1 && W && W->kind == 0) || (R_ == 2 && W && W->kind == 1))                              \
-    launch_learned<HB_, HK_, HE_>(L, F, S, *W, R, g, wg, s, upd);                                     \
+  if ((R_ == 1 && W && W->kind == 0) || (R_ == 2 && W && W->kind == 1)) {                             \
+    if (mf == FORM_NULLV)                                                                             \
+      launch_learned<FORM_NULLV, HB_, HK_, HE_>(L, F, S, *W, R, g, wg, s, upd);                       \
+    else                                                                                              \
+      launch_learned<FORM_FULL, HB_, HK_, HE_>(L, F, S, *W, R, g, wg, s, upd);                        \
+  } else if (persist && mf == FORM_NULLV)                                                             \
+    RQ(FORM_NULLV, R_, HB_, HK_, HE_);                                                                \
   else if (persist)                                                                                   \
-    hipLaunchKernelGGL((k_recover_queue<R_, HB_, HK_, HE_>),                                          \
-                       dim3(resident_groups(k_recover_queue<R_, HB_, HK_, HE_>, R.tile, R.ntiles)), wg, \
-                       0, s, L.k, F, S, R, L.queue);                                                  \
+    RQ(FORM_FULL, R_, HB_, HK_, HE_);                                                                 \
   else if (mf == FORM_POLOIDAL)                                                                       \
     hipLaunchKernelGGL((k_recover<FORM_POLOIDAL, R_, HB_, HK_, HE_>), g, wg, 0, s, L.k, F, S, R);     \
   else if (mf == FORM_FLAT)                                                                           \
@@ -1315,6 +1323,7 @@ int launch_recover(const LaunchCtx &L, const KFields &F, const SharedTabs &S, in
   }
 #undef RC2
 #undef RC
+#undef RQ
   if (rec >= 0 || h) TICK(rec < 0 ? "heating" : h ? "recovery_heating" : "recovery");
   return PG_CHECK_LAUNCH();
 }

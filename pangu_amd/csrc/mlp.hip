@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "../../include/pangu_mlp.h"
+#include "cell_dev.h"
 #include "common.h"
 #include "host.h"
 #include "kernels.h"
@@ -408,10 +409,8 @@ __global__ __launch_bounds__(256) void k_harvest(KCtx C, KFields F, Range3 R, in
     const int64_t id = ((int64_t)k * B.n[1] + j) * B.n[0] + i;
     const int64_t t = ((int64_t)(G.has3d ? k : 0) * G.nj + j) * G.ni + i, ns = G.ncen;
     const auto cen = glb(G.cen);
-    for (int n = 0; n < 16; ++n) {
-      mt[n] = cen[(CG_GCOV + n) * ns + t];
-      mt[16 + n] = cen[(CG_GCON + n) * ns + t];
-    }
+    load_gcov([&](int n) { return cen[n * ns + t]; }, G.nullv, mt);
+    for (int n = 0; n < 16; ++n) mt[16 + n] = cen[(CG_GCON + n) * ns + t];
     mt[32] = cen[CG_SG * ns + t];
     mt[33] = cen[CG_ALPHA * ns + t];
     mt[34] = cen[CG_LAPSE * ns + t];

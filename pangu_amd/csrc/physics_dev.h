@@ -37,7 +37,8 @@ __device__ __forceinline__ double kmin(double a, double b) { return (b < a) ? b 
 // only the entries the form leaves open, and drops the terms whose metric
 // factor is exactly zero: adding +-0 leaves a finite sum unchanged (a sum of
 // zeros may differ in sign), so results equal those of the full sums.
-//   FULL      every entry (any metric: the launch options' kernels);
+//   FULL      every entry (the launch options' kernels, for every metric but
+//             Cartesian Kerr-Schild, whose tables hold no gcov);
 //             g_{0i} = g_{i0} bit for bit
 //   NULLV     eta + xi l l (Cartesian Kerr-Schild): xi and l are read, and
 //             gcov is formed from them as the table was, (xi l_m) l_n
