@@ -242,7 +242,8 @@ __device__ inline double vsq_residual(const double U[9], const CenMetric &m, dou
 // same arguments give the same bits, and each evaluation is a pow, which
 // bounds this scheme (n + 1 of them for n steps; evaluating afresh at the top
 // of every step and after the last takes 2 n + 1).  The divisions run through
-// quot (exact_div.h), as in the 2D scheme, but for the step itself.
+// quot (exact_div.h), as in the 2D scheme, but for the step itself and those by
+// W^2 and W^3.
 template <int MF = FORM_FULL>
 __device__ int c2p_1dvsq(const double U[9], double p[9], double gamma, const CenMetric &m,
                          int &iters, double x0 = -1.0) {
@@ -272,8 +273,11 @@ __device__ int c2p_1dvsq(const double U[9], double p[9], double gamma, const Cen
       const double dWdvsq =
           quot(gamma * (2. - gamma) * pr + (gamma - 1.) * rho, 2. * (gamma - 1.) * (1. - vsq) * (1. - vsq));
       const double fact = (Bsq + Wf);
-      const double resid = Qtsq - vsq * fact * fact + quot(QdotBsq * (Bsq + 2. * Wf), Wsq);
-      const double jac = -fact * (fact + 2. * dWdvsq * (vsq + quot(QdotBsq, W3)));
+      // W^2 and W^3 reach the ends of the exponent range long before the states
+      // do (W^3 is infinite from W = 5.7e102 on, subnormal below 2.8e-103), and
+      // the terms they divide vanish there or stay 0: quot would make them NaN
+      const double resid = Qtsq - vsq * fact * fact + QdotBsq * (Bsq + 2. * Wf) / Wsq;
+      const double jac = -fact * (fact + 2. * dWdvsq * (vsq + QdotBsq / W3));
       const double dx = -resid / jac;
       f = 0.5 * resid * resid;
       df = -2. * f;

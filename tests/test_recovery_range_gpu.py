@@ -1,0 +1,67 @@
+"""1Dvsq recovery of states so thin, or with an entropy so high, that W^3 leaves
+the range of FP64 although the state itself is far inside it: the oracle's
+scheme succeeds, and so does the kernel's, to the same state."""
+import numpy as np
+import pytest
+
+import oracle_py as O
+from pangu_amd import configs
+
+GAMMA = 5.0 / 3.0
+
+
+def _states(n, exps, rng, entropy):
+    """U in the container's form and a guess next to the solution, with u of
+    the order 10^exps, or of order one under an entropy of that order; kept
+    where the oracle's scheme succeeds."""
+    eta = np.diag([-1.0, 1.0, 1.0, 1.0])
+    out = []
+    while len(out) < n:
+        p = np.zeros(10)
+        big = 10.0 ** rng.uniform(*exps)
+        u = 1.0 if entropy else big
+        p[0] = u * rng.uniform(0.5, 2.0)
+        p[1] = u
+        p[2:5] = rng.normal(size=3) * 0.5
+        if entropy or rng.random() < 0.5:
+            p[5:8] = rng.normal(size=3) * np.sqrt(u) * 0.1
+        p[8] = big if entropy else (GAMMA - 1.0) * p[1] * p[0] ** -GAMMA
+        U = O.flux(GAMMA, p, eta, eta, -1.0, 0)[:9]
+        Uh = U.copy()
+        Uh[1] = U[1] - U[0]
+        g = p[:9].copy()
+        g[2:5] *= 0.9
+        if O.c2p(1, Uh, g, GAMMA, eta, eta)[0] == 0:
+            out.append((U, g))
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("exps,entropy", [((-107.0, -103.0), False), ((103.0, 130.0), True), ((-60.0, -20.0), False)])
+def test_onedvsq_outside_the_range_of_w_cubed(exps, entropy):
+    from pangu_amd.sim import HipSim
+    cfg = dict(configs.orszag_tang(32, (2, 1, 1)), recovery=2)
+    sims = [O.OracleSim(cfg), HipSim(cfg)]
+    for s in sims:
+        s.init()
+        s.task("fix_primitive", 0)
+        s.task("conservative", 0)
+    o, h = sims
+    U, P = o.get("cons", 0), o.get("prim", 0)
+    states = _states(48, exps, np.random.default_rng(4), entropy)
+    at = [(n % 2, slice(None), o.s[2], o.s[1] + 2 + n // 4, o.s[0] + 3 + 2 * (n % 4)) for n in range(len(states))]
+    for i, (u, g) in zip(at, states):
+        U[i], P[i] = u, g
+    for s in sims:
+        s.set("cons", U, 1)
+        s.set("prim", P, 1)
+        s.task("recovery", 0, 1)
+    a, b = o.get("prim", 1), h.get("prim", 1).reshape(P.shape)
+    cells = (o.nblocks, 1, o.n[2], o.n[1], o.n[0])
+    got = {f: (o.get(f).reshape(cells), h.get(f).reshape(cells)) for f in ("c2p_status", "c2p_iters")}
+    for i in at:
+        c = (i[0], 0) + i[2:]
+        assert got["c2p_status"][0][c] == 0 and got["c2p_status"][1][c] == 0, i
+        assert abs(int(got["c2p_iters"][0][c]) - int(got["c2p_iters"][1][c])) <= 1, i
+        # pow may differ by an ulp; two Newton ends differ by the tolerance at most
+        assert np.allclose(a[i][:2], b[i][:2], rtol=1e-9, atol=0.0), i
