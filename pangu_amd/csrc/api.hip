@@ -618,7 +618,22 @@ static int build_tables(pangu_ctx *c) {
     }
     if (L.k.dtper == 1 || total >= kDtItems) break;
   }
-  for (int m = 0; m < c->nmesh; ++m) L.maxblocks = std::max(L.maxblocks, c->mfirst[m + 1] - c->mfirst[m]);
+  // lanes per block of the final kernel: the fewest rounds over a mesh's blocks
+  // times passes over a block's items, and of equals the fewest lanes (every
+  // lane goes through the divisions)
+  int64_t least = 0;
+  for (int lanes = 1; lanes <= 64; lanes *= 2) {
+    int64_t most = 0;
+    for (int m = 0; m < c->nmesh; ++m) {
+      const int64_t nb = c->mfirst[m + 1] - c->mfirst[m];
+      const int64_t items = *std::max_element(&dtitems[c->mfirst[m]], &dtitems[c->mfirst[m]] + nb);
+      most = std::max(most, (nb * lanes + 1023) / 1024 * ((items + 4 * lanes - 1) / (4 * lanes)));
+    }
+    if (least == 0 || most < least) {
+      least = most;
+      L.dtlanes = lanes;
+    }
+  }
   const int *db = nullptr, *dfi = nullptr;
   int nd = 0;
   if (int e = upload_tiles(c, dtitems, &db, &dfi, &nd)) return e;

@@ -128,7 +128,7 @@ constexpr int64_t kDtItems = 1024;  // four workgroups per CU
 struct LaunchCtx {
   KCtx k;
   int limiter, riemann, metric, recovery;
-  int maxblocks = 1;               // largest number of blocks of one mesh
+  int dtlanes = 64;                // lanes that share a block's items in k_dt_final
   Range3 interior, entire, face[3], ct;
   Range3 fixx1;  // the entire range in runs of 248 cells (k_fix_flux_x1)
   Range3 x1cells;                  // cell range of the shared-reconstruction X1 sweep

@@ -1101,8 +1101,11 @@ __global__ __launch_bounds__(256) void k_dt_reduce(KCtx C, double *const *alfven
 // estimate) and time += dt.  One workgroup per mesh m: state + 2m = {dt,
 // time}; est_out (optional) + m gets the estimate.  W lanes share a block's
 // items, which the maximum lets them read in any order: the kernel is a few
-// memory round trips long, and one lane walking a block's items made it
-// longer with every item.
+// memory round trips long, one for every 1024 / W blocks and one for every 4 W
+// items of a block, and W is chosen for the fewest (LaunchCtx::dtlanes).  With
+// 16 lanes for every mesh of more than 16 blocks, 512 blocks of 8^3 cells took
+// 23.3 us, 1024 of 8^2 40.7 us and 2000 one-dimensional ones 68 us; with 2, 1
+// and 1 lanes 6.9, 5.4 and 9.2 us; one block of 256^2 cells 4.0 us (64 lanes).
 template <int W>
 __global__ __launch_bounds__(1024) void k_dt_final(KCtx C, const double *red, double *state,
                                                    double dt_factor, double *est_out) {
@@ -1449,12 +1452,12 @@ int launch_dt(const LaunchCtx &L, double *const *alfven, double *red, double *st
   else
     hipLaunchKernelGGL(k_dt_reduce<16>, dim3(L.k.ndt), dim3(256), 0, s, L.k, alfven, red);
   TICK("dt_reduce");
-  // a wavefront per block where no mesh has more than 16 blocks (a single
-  // block may hold hundreds of items), 16 lanes per block otherwise
-  if (L.maxblocks <= 16)
-    hipLaunchKernelGGL(k_dt_final<64>, dim3(L.k.nmesh), dim3(1024), 0, s, L.k, red, state, dt_factor, est_out);
-  else
-    hipLaunchKernelGGL(k_dt_final<16>, dim3(L.k.nmesh), dim3(1024), 0, s, L.k, red, state, dt_factor, est_out);
+#define DF(W)                                                                                              \
+  case W:                                                                                                 \
+    hipLaunchKernelGGL(k_dt_final<W>, dim3(L.k.nmesh), dim3(1024), 0, s, L.k, red, state, dt_factor, est_out); \
+    break;
+  switch (L.dtlanes) { DF(1) DF(2) DF(4) DF(8) DF(16) DF(32) DF(64) }
+#undef DF
   TICK("dt_final");
   return PG_CHECK_LAUNCH();
 }

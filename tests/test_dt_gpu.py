@@ -46,3 +46,37 @@ def test_timestep_estimate_matches_numpy(nx, nb):
         want = min(want, 1.0 / s)
     # dx comes from the mesh generator, not from 1 / nx: a few units in the last place
     assert abs(est[0] - want) <= 8 * np.finfo(np.float64).eps * want
+
+
+# blocks and items of a block that give 1, 1, 2, 4, 8, 16 and 32 lanes to a block
+MANY_BLOCKS = [
+    ((9000, 1, 1), (1500, 1, 1)),
+    ((256, 256, 1), (32, 32, 1)),
+    ((64, 64, 64), (8, 8, 8)),
+    ((48, 48, 48), (6, 6, 6)),
+    ((130, 72, 64), (5, 12, 2)),
+    ((96, 80, 62), (8, 5, 1)),
+    ((640, 640, 1), (5, 5, 1)),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx,nb", MANY_BLOCKS)
+def test_timestep_estimate_of_many_blocks(nx, nb):
+    d = configs.orszag_tang(nx[0], nb)
+    d.update(nx=list(nx), nb=list(nb), enable_heating=0)
+    h = HipSim(d)
+    rng = np.random.default_rng(12)
+    a = rng.uniform(0.0, 1.0, h.get("alfven").shape)
+    a[rng.random(a.shape) < 1e-3] = np.nan
+    h.set("alfven", a)
+    ctx, md, st = h.context()
+    est = (C.c_double * 1)()
+    assert abi.lib().pangu_estimate_timestep(ctx, md[0], est, st) == 0
+    c = np.nanmax(h.interior(a).reshape(h.nblocks, 3, -1), axis=2)
+    want = np.inf
+    for b in range(h.nblocks):
+        dx = h.block_geom(b)[0][3:]
+        q3 = [np.finfo(np.float64).max if nx[q] == 1 else d["cfl"] * dx[q] / c[b, q] for q in range(3)]
+        want = min(want, 1.0 / (1.0 / q3[0] + 1.0 / q3[1] + 1.0 / q3[2]))
+    assert est[0] == want  # the same IEEE operations
