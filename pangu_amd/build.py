@@ -20,7 +20,7 @@ HDF5_ROOT = os.environ.get("PANGU_HDF5_ROOT", "/opt/conda")
 ARCH = os.environ.get("PANGU_OFFLOAD_ARCH", "gfx950")
 
 HOST_SRC = ["geometry.cpp", "problems.cpp", "refine_host.cpp"]
-HIP_SRC = ["kernels.hip", "flux.hip", "sweeps.hip", "api.hip", "sim.hip", "mlp.hip", "diag.hip", "refine.hip"]
+HIP_SRC = ["flux_options.hip", "recovery_options.hip", "kernels.hip", "flux.hip", "sweeps.hip", "api.hip", "sim.hip", "mlp.hip", "diag.hip", "refine.hip"]
 
 # Functions of the host files start on cache lines: by the luck of the layout
 # the initial data of an ensemble of 20 tori took 154 or 178 ms, its tables 33

@@ -20,6 +20,7 @@
 #include "physics_dev.h"
 #include "recovery_dev.h"
 #include "tiles_dev.h"
+#include "update_dev.h"
 
 namespace pangu {
 
@@ -84,214 +85,6 @@ __global__ __launch_bounds__(256) void k_ct_faces(KCtx C, KFields F, double *con
   }
 }
 
-// ------------------------------------ flux divergence, update, source term
-// dU/dt = -[sum_d (A_d F_d(+) - A_d F_d(-))]/V (Parthenon FluxDivergence),
-// U(out) = U(init) + beta dt dU/dt (UpdateIndependentData) and the
-// geometric source U_nu += beta dt sqrt|g| T^r_c Gamma^c_{nu r}
-// (source_term.cc:171-228).  MODE: 1 = divergence only (writes dU/dt),
-// 2 = update only (reads dU/dt), 3 = source only, 4 = all three fused.
-// Flux divergence of one cell (and, for MODE 4, the update from the initial
-// container) with the X2 / X3 terms present when D2 / D3.
-// CTF: the face B fluxes are the constrained-transport values, formed here
-// from edge EMFs that are themselves formed here from the Riemann B fluxes,
-// exactly as k_emf and k_ct_faces would compute them (same operands, same
-// operations), so neither CT kernel runs.  Each cell forms the 12 EMFs on
-// its edges (each edge is shared by four cells; the extra arithmetic is
-// cheaper than a kernel that writes and rereads the EMF arrays).  B
-// components sit at packed indices 5..7.
-template <bool D2, bool D3, int MODE, int NC, bool CTF>
-__device__ __forceinline__ void flux_div(const DevBlock &B, const KFields &F0, const KFields &Finit,
-                                         double *const *dudt, int b,
-                                         int64_t id, int64_t sj, int64_t sk, double bdt,
-                                         double unew[NC]) {
-  const double a1 = B.dx[1] * B.dx[2], a2 = B.dx[0] * B.dx[2], a3 = B.dx[0] * B.dx[1];
-  const double vol = B.dx[0] * B.dx[1] * B.dx[2];
-  const double rvol = 1.0 / vol;
-  double f1p[NC], f1m[NC], f2p[NC], f2m[NC], f3p[NC], f3m[NC], u0[NC];
-  // Every access is base[u + id]: u is a workgroup-uniform offset (a row
-  // sj, a plane sk, or 1) folded into the scalar base, id the cell.
-  const uint32_t id32 = (uint32_t)id;
-  auto at = [&](const double *p, int64_t u) { return ld32(p, u, id32); };
-  // edge EMFs at uniform offset u from the cell, with the k_emf expressions
-  const double *f1b2 = nullptr, *f1b3 = nullptr, *f2b1 = nullptr, *f2b3 = nullptr, *f3b1 = nullptr,
-               *f3b2 = nullptr;
-  if (CTF) {
-    f1b2 = F0.flux[0][b * NC + 6];
-    f1b3 = F0.flux[0][b * NC + 7];
-    if (D2) {
-      f2b1 = F0.flux[1][b * NC + 5];
-      f2b3 = F0.flux[1][b * NC + 7];
-    }
-    if (D3) {
-      f3b1 = F0.flux[2][b * NC + 5];
-      f3b2 = F0.flux[2][b * NC + 6];
-    }
-  }
-  auto E1 = [&](int64_t u) { return 0.25 * ((at(f2b3, u) + at(f2b3, u - sk)) - (at(f3b2, u) + at(f3b2, u - sj))); };
-  auto E2 = [&](int64_t u) { return 0.25 * ((at(f3b1, u) + at(f3b1, u - 1)) - (at(f1b3, u) + at(f1b3, u - sk))); };
-  auto E3 = [&](int64_t u) { return 0.25 * ((at(f1b2, u) + at(f1b2, u - sj)) - (at(f2b1, u) + at(f2b1, u - 1))); };
-#pragma unroll
-  for (int q = 0; q < NC; ++q) {
-    const int c = q - 5;  // B component when CTF and 0 <= c < 3
-    const bool ctb = CTF && c >= 0 && c < 3;
-    const double *f1 = F0.flux[0][b * NC + q];
-    if (ctb && c == 0) {  // normal component: zero
-      f1p[q] = 0;
-      f1m[q] = 0;
-    } else if (ctb && c == 1 && D2) {
-      f1m[q] = 0.5 * (E3(0) + E3(sj));
-      f1p[q] = 0.5 * (E3(1) + E3(1 + sj));
-    } else if (ctb && c == 2 && D3) {
-      f1m[q] = -0.5 * (E2(0) + E2(sk));
-      f1p[q] = -0.5 * (E2(1) + E2(1 + sk));
-    } else {
-      f1p[q] = glb(f1)[id + 1];
-      f1m[q] = glb(f1)[id];
-    }
-    if (D2) {
-      const double *f2 = F0.flux[1][b * NC + q];
-      if (ctb && c == 0) {
-        f2m[q] = -0.5 * (E3(0) + E3(1));
-        f2p[q] = -0.5 * (E3(sj) + E3(sj + 1));
-      } else if (ctb && c == 1) {
-        f2p[q] = 0.;
-        f2m[q] = 0.;
-      } else if (ctb && c == 2 && D3) {
-        f2m[q] = 0.5 * (E1(0) + E1(sk));
-        f2p[q] = 0.5 * (E1(sj) + E1(sj + sk));
-      } else {
-        f2p[q] = at(f2, sj);
-        f2m[q] = at(f2, 0);
-      }
-    }
-    if (D3) {
-      const double *f3 = F0.flux[2][b * NC + q];
-      if (ctb && c == 0) {
-        f3m[q] = 0.5 * (E2(0) + E2(1));
-        f3p[q] = 0.5 * (E2(sk) + E2(sk + 1));
-      } else if (ctb && c == 1 && D2) {
-        f3m[q] = -0.5 * (E1(0) + E1(sj));
-        f3p[q] = -0.5 * (E1(sk) + E1(sk + sj));
-      } else if (ctb && c == 2) {
-        f3p[q] = 0;
-        f3m[q] = 0;
-      } else {
-        f3p[q] = at(f3, sk);
-        f3m[q] = at(f3, 0);
-      }
-    }
-    if (MODE == 4) u0[q] = at(Finit.cons[b * NC + q], 0);
-  }
-#pragma unroll
-  for (int q = 0; q < NC; ++q) {
-    double s = (a1 * f1p[q] - a1 * f1m[q]);
-    if (D2) s += (a2 * f2p[q] - a2 * f2m[q]);
-    if (D3) s += (a3 * f3p[q] - a3 * f3m[q]);
-    const double du = div_by(-s, vol, rvol);
-    if (MODE == 1)
-      glb(dudt[b * NC + q])[id] = du;
-    else
-      unew[q] = u0[q] + bdt * du;
-  }
-}
-
-// Five waves per SIMD is the most the magnetised source-term variants reach
-// without spilling (the field-free ones spill at five and run at four); the
-// kernel is memory bound, so occupancy pays.
-// One cell of k_div_update; the new U also goes to uout (when given).
-// MF: form of the metric for the source term (FORM_FLAT: no source).
-template <int MODE, int MF, bool HB, bool HK, bool CTF>
-__device__ __forceinline__ void div_update_cell(const KCtx &C, const KFields &F0, const KFields &Finit,
-                                                const KFields &F1, double *const *dudt,
-                                                const double *dt_dev, double beta, double bdt_host,
-                                                int b, int k, int j, int i, double *uout) {
-  const DevBlock &B = C.blk[b];
-  const int64_t sj = B.n[0], sk = (int64_t)B.n[0] * B.n[1];
-  const int64_t id = k * sk + j * sj + i;
-  constexpr int NC = ncomp<HB, HK>();
-  const double bdt = dt_dev ? beta * dt_dev[2 * B.mesh] : bdt_host;
-  double unew[NC];
-  if (MODE == 1 || MODE == 4) {
-    // one uniform branch on the block's active dimensions, so the loads of
-    // all components sit in one basic block and overlap
-    const bool d2 = B.n[1] > 1, d3 = B.n[2] > 1;
-    if (d2 && d3)
-      flux_div<true, true, MODE, NC, CTF>(B, F0, Finit, dudt, b, id, sj, sk, bdt, unew);
-    else if (d2)
-      flux_div<true, false, MODE, NC, CTF>(B, F0, Finit, dudt, b, id, sj, sk, bdt, unew);
-    else if (d3)
-      flux_div<false, true, MODE, NC, CTF>(B, F0, Finit, dudt, b, id, sj, sk, bdt, unew);
-    else
-      flux_div<false, false, MODE, NC, CTF>(B, F0, Finit, dudt, b, id, sj, sk, bdt, unew);
-  } else if (MODE == 2) {
-#pragma unroll
-    for (int q = 0; q < NC; ++q)
-      unew[q] = glb(Finit.cons[b * NC + q])[id] + bdt * glb(dudt[b * NC + q])[id];
-  } else {
-#pragma unroll
-    for (int q = 0; q < NC; ++q) unew[q] = glb(F1.cons[b * NC + q])[id];
-  }
-  if (MODE == 1) return;
-  if (MF != FORM_FLAT && (MODE == 3 || MODE == 4)) {
-    const DevGeo &G = C.geo[B.geo];
-    const int64_t t = cen_index(G, k, j, i);
-    CenLoad m;
-    load_cen_state<MF>(G, t, m);
-    double p[NPRIM];
-#pragma unroll
-    for (int s = 0; s < NPRIM; ++s) p[s] = 0.0;
-#pragma unroll
-    for (int q = 0; q < NC; ++q) p[slot_of<HB, HK>(q)] = glb(F1.prim[b * NC + q])[id];
-    St s;
-    calc_state<MF, HB>(p, m.g, m.gc0, m.alpha, s);
-    const double gam = C.ph.gamma;
-    const double pg = (gam - 1.) * p[ENY];
-    const double h = p[RHO] + gam * p[ENY];
-    const double etot = HB ? h + s.bsq : h, ptot = HB ? pg + 0.5 * s.bsq : pg;
-    double T[4][4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      T[0][c] = tmunu<0, HB>(s, etot, ptot, c);
-      T[1][c] = tmunu<1, HB>(s, etot, ptot, c);
-      T[2][c] = tmunu<2, HB>(s, etot, ptot, c);
-      T[3][c] = tmunu<3, HB>(s, etot, ptot, c);
-    }
-    // one scalar base for the connection block (40 or 64 slots) and a
-    // 32-bit index per slot: per-slot scalar bases would exhaust the scalar
-    // registers
-    const double *conn = G.cen + (int64_t)CG_CONN * G.ncen;
-    const uint32_t ncen32 = (uint32_t)G.ncen, t32 = (uint32_t)t;
-    const bool sym = G.conn_sym != 0;
-#pragma unroll
-    for (int dd = 0; dd < 4; ++dd) {
-      double con = 0.0;
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int slot = sym ? 10 * c + conn_pair(dd, r) : 16 * c + 4 * dd + r;
-          con += T[r][c] * ldc32(conn, 0, (uint32_t)slot * ncen32 + t32);
-        }
-      const int q = (dd == 0) ? 1 : 1 + dd;
-      unew[q] += con * m.sg * bdt;
-    }
-  }
-  if (uout) {
-    // the caller goes on with the values; memory is next read a stage later
-#pragma unroll
-    for (int q = 0; q < NC; ++q) {
-      stnt32(F1.cons[b * NC + q], (uint32_t)id, unew[q]);
-      uout[q] = unew[q];
-    }
-  } else {
-    // the next kernel (the source term, the recovery) reads them: with stores
-    // past L2 the tasks from flux divergence to source took 53.1 us for 64^3
-    // cells in MKS instead of 50.1
-#pragma unroll
-    for (int q = 0; q < NC; ++q) glb(F1.cons[b * NC + q])[id] = unew[q];
-  }
-}
-
 template <int MODE, int MF, bool HB, bool HK, bool CTF>
 __global__ __launch_bounds__(256, (HB && MODE != 1) ? 5 : 4) void k_div_update(KCtx C, KFields F0, KFields Finit, KFields F1,
                                                     double *const *dudt,
@@ -301,209 +94,6 @@ __global__ __launch_bounds__(256, (HB && MODE != 1) ? 5 : 4) void k_div_update(K
   if (!decode_tile(C, R, b, k, j, i)) return;
   div_update_cell<MODE, MF, HB, HK, CTF>(C, F0, Finit, F1, dudt, dt_dev, beta, bdt_host, b, k, j, i,
                                           nullptr);
-}
-
-// -------------------------------------------------- recovery (+ heating)
-// ApplyElectronHeating (electron_heating.cc:66-109) on one recovered cell
-// from its primitives p (rho, u, u~, B and the stale entropy; K_e is not
-// read); the centre metric is loaded here.
-template <int MF, bool HB, bool HK>
-__device__ __forceinline__ void heat_vals(const KCtx &C, const KFields &F, const DevGeo &G, int64_t t,
-                                          int b, int64_t id, const Arr32<double> *pp,
-                                          const double p[NPRIM], const double *ureg = nullptr) {
-  constexpr int NC = ncomp<HB, HK>();
-  CenLoad m;
-  load_cen_state<MF>(G, t, m);
-  St s;
-  calc_state<MF, HB>(p, m.g, m.gc0, m.alpha, s);
-  const uint32_t id32 = (uint32_t)id;
-  // conserved components: from memory, or from registers (ureg, in
-  // component order) when the caller has just written them
-  auto cu = [&](int q) { return ureg ? ureg[q] : ld32(F.cons[b * NC + q], 0, id32); };
-  const double crho = cu(0);
-  HeatIn c;
-  c.rho = p[RHO];
-  c.energy = p[ENY];
-  c.bsq = s.bsq;
-  c.adv_total = cu(ient<HB>()) / crho;
-  c.rec_total = p[ENT];
-  c.adv_e = cu(ikel<HB>()) / crho;
-  pp[ikel<HB>()][id] = heat_apply(C.ph, c);
-}
-
-// The same with the primitives read from memory.
-template <int MF, bool HB, bool HK>
-__device__ __forceinline__ void heat_cell(const KCtx &C, const KFields &F, const DevGeo &G, int64_t t,
-                                          int b, int64_t id, const Arr32<double> *pp) {
-  constexpr int NC = ncomp<HB, HK>();
-  double p[NPRIM];
-#pragma unroll
-  for (int s = 0; s < NPRIM; ++s) p[s] = 0.0;
-#pragma unroll
-  for (int q = 0; q < NC; ++q) p[slot_of<HB, HK>(q)] = pp[q][id];
-  heat_vals<MF, HB, HK>(C, F, G, t, b, id, pp, p);
-}
-
-// The centre metric the recovery reads, as far as form MF leaves it open
-// (gcon is not symmetric bit for bit, so each open entry is read), sqrt|g|
-// and 1/sqrt(-g^00).
-template <int MF>
-__device__ __forceinline__ void load_cen_metric(const DevGeo &G, int64_t t, CenMetric &m, double &sg,
-                                                double &alpha) {
-  auto comp = [&](int n) { return ldc32(G.cen, (int64_t)n * G.ncen, (uint32_t)t); };
-  double gc0[4];
-  load_metric<MF, CG_GCON, CG_ALPHA>(comp, m.gcov, gc0, alpha);
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      m.gcon[4 * r + c] = MF == FORM_FLAT ? m.gcov[4 * r + c] : g_open<MF>(r, c) ? comp(CG_GCON + 4 * r + c) : 0.0;
-  m.lapse = MF == FORM_FLAT ? 1.0 : comp(CG_LAPSE);
-  sg = MF == FORM_FLAT ? 1.0 : comp(CG_SG);
-}
-
-// Recovery (invertor.cc:184-319) and, when HEAT, ApplyElectronHeating
-// (electron_heating.cc:66-109) on the recovered cell.  REC: 0 chainer,
-// 1 Kastaun, 2 1Dvsq alone, -1 none (heating only).
-template <int MF, int REC, bool HB, bool HK, bool HEAT>
-__device__ __forceinline__ void recover_cell(const KCtx &C, const KFields &F, const SharedTabs &S, int b,
-                                             int k, int j, int i, double x0 = -1.0,
-                                             const double *ureg = nullptr) {
-  const DevBlock &B = C.blk[b];
-  const int64_t id = ((int64_t)k * B.n[1] + j) * B.n[0] + i;
-  constexpr int NC = ncomp<HB, HK>();
-  const DevGeo &G = C.geo[B.geo];
-  const int64_t t = cen_index(G, k, j, i);
-  const Phys &P = C.ph;
-  Arr32<double> pp[NC];
-#pragma unroll
-  for (int q = 0; q < NC; ++q) pp[q] = Arr32<double>{F.prim[b * NC + q]};
-  if (REC >= 0) {
-    const bool chainer = (REC != 1);
-    bool excised = false;
-    if (P.metric == PANGU_METRIC_CKS && ldc32(G.cen, (int64_t)CG_RAD * G.ncen, (uint32_t)t) < P.r_excise) excised = true;
-    if (excised) {
-      if (chainer && S.flag) glb(S.flag[b])[id] = 0.0;
-      if (S.status) glb(S.status[b])[id] = -1;
-      if (S.iters) glb(S.iters[b])[id] = 0;
-    } else {
-      CenMetric m;
-      double sg, alpha;
-      load_cen_metric<MF>(G, t, m, sg, alpha);
-      double U[9], Ph[9], bnew[3] = {0.0, 0.0, 0.0};
-      Arr32<double> cons[NC];
-#pragma unroll
-      for (int q = 0; q < NC; ++q) cons[q] = Arr32<double>{F.cons[b * NC + q]};
-      // U from memory, or from registers (ureg) when the update just wrote it
-      auto cv = [&](int q) { return ureg ? ureg[q] : (double)cons[q][id]; };
-      const double c_rho = cv(0), c_eny = cv(1);
-      const double isg = 1.0 / sg;
-      const double aos = alpha * isg;
-      U[RHO] = aos * c_rho;
-      U[ENY] = aos * (c_eny - c_rho);
-      U[UX1] = aos * cv(2);
-      U[UX2] = aos * cv(3);
-      U[UX3] = aos * cv(4);
-      if (HB) {
-        const double cb1 = cv(5), cb2 = cv(6), cb3 = cv(7);
-        U[BX1] = aos * cb1;
-        U[BX2] = aos * cb2;
-        U[BX3] = aos * cb3;
-        bnew[0] = cb1 * isg;
-        bnew[1] = cb2 * isg;
-        bnew[2] = cb3 * isg;
-        pp[5][id] = bnew[0];
-        pp[6][id] = bnew[1];
-        pp[7][id] = bnew[2];
-      } else {
-        U[BX1] = 0.0;
-        U[BX2] = 0.0;
-        U[BX3] = 0.0;
-      }
-      U[ENT] = aos * cv(ient<HB>());
-      // the Newton schemes start from the previous primitives; Kastaun's
-      // bracket needs none (it writes rho, u and u~ only on success), so
-      // their loads are skipped
-#pragma unroll
-      for (int s = 0; s < 9; ++s) Ph[s] = 0.0;
-      if (REC != 1) {
-        Ph[RHO] = pp[0][id];
-        Ph[ENY] = pp[1][id];
-        Ph[UX1] = pp[2][id];
-        Ph[UX2] = pp[3][id];
-        Ph[UX3] = pp[4][id];
-        Ph[ENT] = pp[ient<HB>()][id];
-      }
-      int st = 0, it = 0, itn = 0;
-      bool write = true;
-      if (REC == 1) {
-        double mu = 0.0;
-        st = c2p_kastaun<MF>(U, Ph, P.gamma, m, it, &mu);
-        if (S.root) glb(S.root[b])[id] = (st == 0) ? mu : __builtin_nan("");
-        itn = it;
-        write = (st == 0);
-      } else if (REC == 2) {
-        // x0 >= 0: the learned start (k_recover_learned_vsq)
-        st = c2p_1dvsq<MF>(U, Ph, P.gamma, m, it, x0);
-        itn = it;
-      } else {
-        st = c2p_2d<MF>(U, Ph, P.gamma, m, it);
-        itn = it;
-        if (st != 0) {
-          st = c2p_1dvsq<MF>(U, Ph, P.gamma, m, it);
-          itn += it;
-          if (st != 0) {
-            st = c2p_1d<MF>(U, Ph, P.gamma, m, it);
-            itn += it;
-          }
-        }
-      }
-      if (chainer && S.flag) {
-        const double fv = (st == 0) ? 1.0 : 0.0;
-        glb(S.flag[b])[id] = fv;
-        if (S.flag_rec) glb(S.flag_rec[b])[id] = fv;
-      }
-      if (S.status) glb(S.status[b])[id] = st;
-      if (S.iters) glb(S.iters[b])[id] = itn;
-      if (write) {
-        pp[0][id] = Ph[RHO];
-        pp[1][id] = Ph[ENY];
-        pp[2][id] = Ph[UX1];
-        pp[3][id] = Ph[UX2];
-        pp[4][id] = Ph[UX3];
-      }
-      if (HEAT && HK) {
-        // the heating reads the primitives just written from registers (the
-        // compiler cannot forward them: the stores may alias other arrays);
-        // a cell whose recovery failed keeps its previous primitives
-        double hp[NPRIM];
-#pragma unroll
-        for (int s = 0; s < NPRIM; ++s) hp[s] = 0.0;
-        if (write) {
-          hp[RHO] = Ph[RHO];
-          hp[ENY] = Ph[ENY];
-          hp[UX1] = Ph[UX1];
-          hp[UX2] = Ph[UX2];
-          hp[UX3] = Ph[UX3];
-        } else {
-          hp[RHO] = pp[0][id];
-          hp[ENY] = pp[1][id];
-          hp[UX1] = pp[2][id];
-          hp[UX2] = pp[3][id];
-          hp[UX3] = pp[4][id];
-        }
-        if (HB) {
-          hp[BX1] = bnew[0];
-          hp[BX2] = bnew[1];
-          hp[BX3] = bnew[2];
-        }
-        hp[ENT] = pp[ient<HB>()][id];
-        heat_vals<MF, HB, HK>(C, F, G, t, b, id, pp, hp, ureg);
-        return;
-      }
-    }
-  }
-  if (HEAT && HK) heat_cell<MF, HB, HK>(C, F, G, t, b, id, pp);
 }
 
 template <int MF, int REC, bool HB, bool HK, bool HEAT>
@@ -535,247 +125,6 @@ __global__ __launch_bounds__(256) void k_update_recover(KCtx C, KFields F0, KFie
   double u[NPRIM];
   div_update_cell<4, MF, HB, HK, CTF>(C, F0, Finit, F1, nullptr, dt_dev, beta, bdt_host, b, k, j, i, u);
   recover_cell<MF, REC, HB, HK, HEAT>(C, F1, S, b, k, j, i, -1.0, u);
-}
-
-// Persistent form of k_recover: a grid no larger than what the GPU holds
-// at once pulls tiles from a queue (queue[0]: next tile, queue[1]:
-// workgroups done) until every tile is taken; the last workgroup out resets
-// the queue for the next launch on the stream, so a captured graph replays
-// it without a memset.  Tiles carry no dependencies, so no workgroup ever
-// waits for another.  Same cells, same arithmetic: identical results.
-template <int MF, int REC, bool HB, bool HK, bool HEAT>
-__global__ __launch_bounds__(256) void k_recover_queue(KCtx C, KFields F, SharedTabs S, Range3 R,
-                                                       unsigned *queue) {
-  __shared__ int tile_sh;
-  for (;;) {
-    if (threadIdx.x == 0) tile_sh = (int)atomicAdd(&queue[0], 1u);
-    __syncthreads();
-    const int T = tile_sh;
-    __syncthreads();  // every thread has read the tile before the next pull
-    if (T >= R.ntiles) break;
-    int b, k, j, i;
-    if (decode_tile_at(C, R, T, b, k, j, i)) recover_cell<MF, REC, HB, HK, HEAT>(C, F, S, b, k, j, i);
-  }
-  if (threadIdx.x == 0 && atomicAdd(&queue[1], 1u) == gridDim.x - 1) {
-    atomicExch(&queue[0], 0u);
-    atomicExch(&queue[1], 0u);
-  }
-}
-
-// Kastaun recovery with the learned starting bracket (and, when HEAT, the
-// electron heating): k_recover<1, ...> whose wavefronts that hold a cell
-// passing the gate (its previous recovery took at least S.gate
-// false-position steps) run the network on the matrix cores inside the
-// wavefront (wave_mlp); every cell of such a wavefront then starts the
-// search from the prediction (kastaun_guess_k), the others search [0, 1]
-// as k_recover does.  Status, iteration and field outputs are those of
-// k_recover; the recovered state agrees with it to the solver tolerance
-// (another false-position path to a root of the same function), not bit for
-// bit.
-template <int MF, bool HB, bool HK>
-__device__ __forceinline__ int learned_setup(const KCtx &C, const KFields &F, const DevGeo &G, int64_t t,
-                                             int b, int64_t id, KastaunIn &kin) {
-  constexpr int NC = ncomp<HB, HK>();
-  const int64_t ns = G.ncen;
-  CenMetric m;
-  auto comp = [&](int n) { return ldc32(G.cen, (int64_t)n * ns, (uint32_t)t); };
-  if (MF == FORM_NULLV)
-    gcov_from_null(comp, m.gcov);
-  else
-    load_gcov(comp, 0, m.gcov);
-#pragma unroll
-  for (int n = 0; n < 16; ++n) m.gcon[n] = comp(CG_GCON + n);
-  m.lapse = ldc32(G.cen, (int64_t)CG_LAPSE * ns, (uint32_t)t);
-  const double aos = ldc32(G.cen, (int64_t)CG_ALPHA * ns, (uint32_t)t) * (1.0 / ldc32(G.cen, (int64_t)CG_SG * ns, (uint32_t)t));
-  const double *const *cons = F.cons + (int64_t)b * NC;
-  const double c_rho = glb(cons[0])[id], c_eny = glb(cons[1])[id];
-  double U[9];
-  U[RHO] = aos * c_rho;
-  U[ENY] = aos * (c_eny - c_rho);
-  U[UX1] = aos * glb(cons[2])[id];
-  U[UX2] = aos * glb(cons[3])[id];
-  U[UX3] = aos * glb(cons[4])[id];
-#pragma unroll
-  for (int a = 0; a < 3; ++a) U[BX1 + a] = HB ? aos * glb(cons[5 + a])[id] : 0.0;
-  U[ENT] = aos * glb(cons[ient<HB>()])[id];
-  return kastaun_setup(U, m, kin);
-}
-
-// UPD 1 or 2: the cell's update (k_div_update mode 4; 2 with the source)
-// runs first, as in k_update_recover; the recovery then reads the U this
-// thread has just stored.
-template <int MF, bool HB, bool HK, bool HEAT, int UPD>
-__global__ __launch_bounds__(256) void k_recover_learned(KCtx C, KFields F, SharedTabs S, MlpFrag W,
-                                                         Range3 R, UpdArgs A) {
-  int b = 0, k = 0, j = 0, i = 0;
-  const bool cell = decode_tile(C, R, b, k, j, i);  // false on the whole workgroup past the range
-  if (UPD && cell)
-    div_update_cell<4, UPD == 2 ? MF : FORM_FLAT, HB, HK, HB>(C, A.F0, A.Finit, F, nullptr, A.dt_dev, A.beta, A.bdt_host, b,
-                                             k, j, i, nullptr);
-  const int lane = threadIdx.x & 63;
-  constexpr int NC = ncomp<HB, HK>();
-  const Phys &P = C.ph;
-  const DevBlock &B = C.blk[cell ? b : 0];
-  const DevGeo &G = C.geo[B.geo];
-  const int64_t id = cell ? ((int64_t)k * B.n[1] + j) * B.n[0] + i : 0;
-  const int64_t t = cell ? cen_index(G, k, j, i) : 0;
-  const bool active =
-      cell && !(P.metric == PANGU_METRIC_CKS && ldc32(G.cen, (int64_t)CG_RAD * G.ncen, (uint32_t)t) < P.r_excise);
-  // The workgroup votes on the previous iteration counts alone, before any
-  // other load: a workgroup with no cell passing the gate then runs as
-  // k_recover<1> does, with no further barrier.  The network's cost is per
-  // wavefront, so a wavefront that runs it for a gated cell serves every
-  // cell of it with a valid setup.
-  int prev = 0;
-  if (active && S.iters) prev = glb(S.iters[b])[id];
-  const bool gated = active && S.iters && prev >= S.gate;
-  KastaunIn kin;
-  int setup = -1;
-  double guess = -1.0;
-  __shared__ MlpLds lds;
-  // every thread of the workgroup reaches the vote (no early return above)
-  if (__syncthreads_or(gated)) {
-    mlp_stage(W, lds, threadIdx.x, blockDim.x);
-    if (active) setup = learned_setup<MF, HB, HK>(C, F, G, t, b, id, kin);
-    __syncthreads();
-    const bool want = setup == 0;
-    if (__ballot(gated && want)) {  // uniform over the wavefront: all 64 lanes run the network
-      float x[5] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-      if (want) {
-        float f[5];
-        c2p_features(kin, f);
-#pragma unroll
-        for (int q = 0; q < 5; ++q) x[q] = bf2f(f2bf((f[q] - W.mean[q]) / W.dev[q]));
-      }
-      const float z = wave_mlp(lds, W.b4[0], x, lane);
-      if (want) guess = (double)(1.0f / (1.0f + expf(-z)));
-      // the setup is recomputed from memory (same inputs, same bits)
-      // instead of being held in registers across the network
-      __asm__ volatile("" ::: "memory");
-      if (active) setup = learned_setup<MF, HB, HK>(C, F, G, t, b, id, kin);
-    }
-  } else if (active) {
-    setup = learned_setup<MF, HB, HK>(C, F, G, t, b, id, kin);
-  }
-  if (!cell) return;
-  Arr32<double> pp[NC];
-#pragma unroll
-  for (int q = 0; q < NC; ++q) pp[q] = Arr32<double>{F.prim[b * NC + q]};
-  if (!active) {
-    if (S.status) glb(S.status[b])[id] = -1;
-    if (S.iters) glb(S.iters[b])[id] = 0;
-  } else {
-    double bnew[3] = {0.0, 0.0, 0.0};
-    if (HB) {
-      const double isg = 1.0 / ldc32(G.cen, (int64_t)CG_SG * G.ncen, (uint32_t)t);
-#pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        bnew[a] = glb(F.cons[b * NC + 5 + a])[id] * isg;
-        pp[5 + a][id] = bnew[a];
-      }
-    }
-    double Ph[9];
-    double mu = 0.0;
-    int st, it = 0;
-    if (setup != 0) {
-      st = setup;
-    } else {
-      // one code path: without a guess (-1) kastaun_guess_k searches [0, 1]
-      // exactly as kastaun_plain_k does
-      int ev = 0;
-      st = kastaun_guess_k(kin, P.gamma, Ph, guess, S.delta, it, ev, &mu);
-    }
-    if (S.root) glb(S.root[b])[id] = (st == 0) ? mu : __builtin_nan("");
-    if (S.status) glb(S.status[b])[id] = st;
-    if (S.iters) glb(S.iters[b])[id] = it;
-    if (st == 0) {
-      pp[0][id] = Ph[RHO];
-      pp[1][id] = Ph[ENY];
-      pp[2][id] = Ph[UX1];
-      pp[3][id] = Ph[UX2];
-      pp[4][id] = Ph[UX3];
-    }
-    if (HEAT && HK) {
-      // as recover_cell: the heating takes the primitives just written from
-      // registers (a failed cell keeps its previous ones, from memory)
-      double hp[NPRIM];
-#pragma unroll
-      for (int q = 0; q < NPRIM; ++q) hp[q] = 0.0;
-      if (st == 0) {
-        hp[RHO] = Ph[RHO];
-        hp[ENY] = Ph[ENY];
-        hp[UX1] = Ph[UX1];
-        hp[UX2] = Ph[UX2];
-        hp[UX3] = Ph[UX3];
-      } else {
-        hp[RHO] = pp[0][id];
-        hp[ENY] = pp[1][id];
-        hp[UX1] = pp[2][id];
-        hp[UX2] = pp[3][id];
-        hp[UX3] = pp[4][id];
-      }
-      if (HB) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) hp[BX1 + a] = bnew[a];
-      }
-      hp[ENT] = pp[ient<HB>()][id];
-      heat_vals<MF, HB, HK>(C, F, G, t, b, id, pp, hp);
-      return;
-    }
-  }
-  if (HEAT && HK) heat_cell<MF, HB, HK>(C, F, G, t, b, id, pp);
-}
-
-// The 1Dvsq recovery with the learned start (and, when HEAT, the heating):
-// the vote, the staging and the in-wave network of k_recover_learned, on
-// the same features (the Kastaun invariants of the cell's U and metric),
-// predicting z = log u^2; every cell of a wavefront that ran the network
-// then starts its Newton iteration from v^2 = u^2 / (1 + u^2) =
-// logistic(z) instead of the previous primitives' v^2.  Everything else is
-// recover_cell<2>: the result agrees with k_recover<2> to the Newton
-// tolerance, not bit for bit.
-template <int MF, bool HB, bool HK, bool HEAT, int UPD>
-__global__ __launch_bounds__(256) void k_recover_learned_vsq(KCtx C, KFields F, SharedTabs S, MlpFrag W,
-                                                             Range3 R, UpdArgs A) {
-  int b = 0, k = 0, j = 0, i = 0;
-  const bool cell = decode_tile(C, R, b, k, j, i);  // false on the whole workgroup past the range
-  if (UPD && cell)
-    div_update_cell<4, UPD == 2 ? MF : FORM_FLAT, HB, HK, HB>(C, A.F0, A.Finit, F, nullptr, A.dt_dev, A.beta, A.bdt_host, b,
-                                             k, j, i, nullptr);
-  const int lane = threadIdx.x & 63;
-  const Phys &P = C.ph;
-  const DevBlock &B = C.blk[cell ? b : 0];
-  const DevGeo &G = C.geo[B.geo];
-  const int64_t id = cell ? ((int64_t)k * B.n[1] + j) * B.n[0] + i : 0;
-  const int64_t t = cell ? cen_index(G, k, j, i) : 0;
-  const bool active =
-      cell && !(P.metric == PANGU_METRIC_CKS && ldc32(G.cen, (int64_t)CG_RAD * G.ncen, (uint32_t)t) < P.r_excise);
-  int prev = 0;
-  if (active && S.iters) prev = glb(S.iters[b])[id];
-  const bool gated = active && S.iters && prev >= S.gate;
-  double x0 = -1.0;
-  __shared__ MlpLds lds;
-  // every thread of the workgroup reaches the vote (no early return above)
-  if (__syncthreads_or(gated)) {
-    mlp_stage(W, lds, threadIdx.x, blockDim.x);
-    KastaunIn kin;
-    const int setup = active ? learned_setup<MF, HB, HK>(C, F, G, t, b, id, kin) : -1;
-    __syncthreads();
-    const bool want = setup == 0;
-    if (__ballot(gated && want)) {  // uniform over the wavefront: all 64 lanes run the network
-      float x[5] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-      if (want) {
-        float f[5];
-        c2p_features(kin, f);
-#pragma unroll
-        for (int q = 0; q < 5; ++q) x[q] = bf2f(f2bf((f[q] - W.mean[q]) / W.dev[q]));
-      }
-      const float z = wave_mlp(lds, W.b4[0], x, lane);
-      if (want) x0 = (double)(1.0f / (1.0f + expf(-z)));
-    }
-  }
-  if (!cell) return;
-  recover_cell<MF, 2, HB, HK, HEAT>(C, F, S, b, k, j, i, x0);
 }
 
 // ---------------------------------------------------------- FixRecovery
@@ -1167,19 +516,6 @@ __global__ __launch_bounds__(1024) void k_dt_final(KCtx C, const double *red, do
 }
 
 // ===================================================================== host
-// Grid of a persistent kernel: the workgroups the GPU holds at once (at
-// most ntiles), so every workgroup runs from the start.
-template <typename K>
-static int resident_groups(K kernel, int threads, int ntiles) {
-  int dev = 0, per_cu = 0, ncu = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0) != hipSuccess ||
-      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return 1;
-  const int64_t n = (int64_t)(per_cu > 0 ? per_cu : 1) * (ncu > 0 ? ncu : 1);
-  return (int)(n < ntiles ? n : ntiles);
-}
-
 hipError_t KernelClock::mark(const char *name, hipStream_t s) {
   if (n == events.size()) {
     hipEvent_t e;
@@ -1263,28 +599,6 @@ int launch_div_update(const LaunchCtx &L, int mode, const KFields &F0, const KFi
   return PG_CHECK_LAUNCH();
 }
 
-template <int MF, bool HB, bool HK, bool HEAT>
-static void launch_learned(const LaunchCtx &L, const KFields &F, const SharedTabs &S, const MlpFrag &W,
-                           const Range3 &R, dim3 g, dim3 wg, hipStream_t s, const UpdArgs *upd) {
-  const UpdArgs A = upd ? *upd : UpdArgs{};
-  const int u = !upd ? 0 : (L.metric != PANGU_METRIC_MINKOWSKI ? 2 : 1);
-  if (W.kind == 0) {
-    if (u == 2)
-      hipLaunchKernelGGL((k_recover_learned<MF, HB, HK, HEAT, 2>), g, wg, 0, s, L.k, F, S, W, R, A);
-    else if (u == 1)
-      hipLaunchKernelGGL((k_recover_learned<MF, HB, HK, HEAT, 1>), g, wg, 0, s, L.k, F, S, W, R, A);
-    else
-      hipLaunchKernelGGL((k_recover_learned<MF, HB, HK, HEAT, 0>), g, wg, 0, s, L.k, F, S, W, R, A);
-  } else {
-    if (u == 2)
-      hipLaunchKernelGGL((k_recover_learned_vsq<MF, HB, HK, HEAT, 2>), g, wg, 0, s, L.k, F, S, W, R, A);
-    else if (u == 1)
-      hipLaunchKernelGGL((k_recover_learned_vsq<MF, HB, HK, HEAT, 1>), g, wg, 0, s, L.k, F, S, W, R, A);
-    else
-      hipLaunchKernelGGL((k_recover_learned_vsq<MF, HB, HK, HEAT, 0>), g, wg, 0, s, L.k, F, S, W, R, A);
-  }
-}
-
 int launch_recover(const LaunchCtx &L, const KFields &F, const SharedTabs &S, int rec, bool heat,
                    const MlpFrag *W, hipStream_t s, const UpdArgs *upd) {
   // a fused update needs the learned kernel of the scheme (k_update_recover
@@ -1297,44 +611,38 @@ int launch_recover(const LaunchCtx &L, const KFields &F, const SharedTabs &S, in
   const bool hb = L.k.iBX >= 0, hk = L.k.iKEL >= 0;
   const bool persist = L.persist_recovery && L.queue;
   const int mf = metric_form(L.metric);
-#define RQ(MF_, R_, HB_, HK_, HE_)                                                                    \
-  hipLaunchKernelGGL((k_recover_queue<MF_, R_, HB_, HK_, HE_>),                                       \
-                     dim3(resident_groups(k_recover_queue<MF_, R_, HB_, HK_, HE_>, R.tile, R.ntiles)), \
-                     wg, 0, s, L.k, F, S, R, L.queue)
 #define RC(R_, HB_, HK_, HE_)                                                                        \
-  if ((R_ == 1 && W && W->kind == 0) || (R_ == 2 && W && W->kind == 1)) {                             \
-    if (mf == FORM_NULLV)                                                                             \
-      launch_learned<FORM_NULLV, HB_, HK_, HE_>(L, F, S, *W, R, g, wg, s, upd);                       \
-    else                                                                                              \
-      launch_learned<FORM_FULL, HB_, HK_, HE_>(L, F, S, *W, R, g, wg, s, upd);                        \
-  } else if (persist && mf == FORM_NULLV)                                                             \
-    RQ(FORM_NULLV, R_, HB_, HK_, HE_);                                                                \
-  else if (persist)                                                                                   \
-    RQ(FORM_FULL, R_, HB_, HK_, HE_);                                                                 \
-  else if (mf == FORM_POLOIDAL)                                                                       \
+  if (mf == FORM_POLOIDAL)                                                                            \
     hipLaunchKernelGGL((k_recover<FORM_POLOIDAL, R_, HB_, HK_, HE_>), g, wg, 0, s, L.k, F, S, R);     \
   else if (mf == FORM_FLAT)                                                                           \
     hipLaunchKernelGGL((k_recover<FORM_FLAT, R_, HB_, HK_, HE_>), g, wg, 0, s, L.k, F, S, R);         \
   else                                                                                                \
     hipLaunchKernelGGL((k_recover<FORM_NULLV, R_, HB_, HK_, HE_>), g, wg, 0, s, L.k, F, S, R)
-#define RC2(R_, HE_)                          \
-  if (hb && hk) { RC(R_, true, true, HE_); }  \
-  else if (hb) { RC(R_, true, false, HE_); }  \
-  else if (hk) { RC(R_, false, true, HE_); }  \
-  else { RC(R_, false, false, HE_); }
+// (heating comes with K_e)
+#define RC2(R_)                                  \
+  if (hb && h) { RC(R_, true, true, true); }     \
+  else if (h) { RC(R_, false, true, true); }     \
+  else if (hb && hk) { RC(R_, true, true, false); } \
+  else if (hb) { RC(R_, true, false, false); }   \
+  else if (hk) { RC(R_, false, true, false); }   \
+  else { RC(R_, false, false, false); }
   const bool h = heat && hk;
-  if (rec == 0) {
-    if (h) { RC2(0, true) } else { RC2(0, false) }
+  const bool learned = W && ((rec == 1 && W->kind == 0) || (rec == 2 && W->kind == 1));
+  if (learned || persist) {
+    launch_recover_option(L, F, S, rec, h, learned ? W : nullptr, R, s, upd);
+  } else if (rec == 0) {
+    RC2(0)
   } else if (rec == 1) {
-    if (h) { RC2(1, true) } else { RC2(1, false) }
+    RC2(1)
   } else if (rec == 2) {
-    if (h) { RC2(2, true) } else { RC2(2, false) }
+    RC2(2)
+  } else if (h && hb) {
+    RC(-1, true, true, true);
   } else if (h) {
-    RC2(-1, true)
+    RC(-1, false, true, true);
   }
 #undef RC2
 #undef RC
-#undef RQ
   if (rec >= 0 || h) TICK(rec < 0 ? "heating" : h ? "recovery_heating" : "recovery");
   return PG_CHECK_LAUNCH();
 }

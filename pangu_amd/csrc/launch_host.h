@@ -21,6 +21,14 @@ inline Range3 family_range(const LaunchCtx &L, int id, const Range3 &base, int f
   return R;
 }
 
+// Recovery with the learned start of W or, without a model, as a persistent
+// work queue (recovery_options.hip); heat only where there is K_e.
+void launch_recover_option(const LaunchCtx &L, const KFields &F, const SharedTabs &S, int rec, bool heat,
+                           const MlpFrag *W, const Range3 &R, hipStream_t s, const UpdArgs *upd);
+// The sweep along dir in one of its other forms (flux_options.hip).  0: the
+// plain form is asked for; 1: launched; -1: nothing to launch.
+int launch_sweep_option(const LaunchCtx &L, int dir, const KFields &F, double *const *alfven, hipStream_t s);
+
 #define PG_CHECK_LAUNCH() (hipGetLastError() == hipSuccess ? 0 : -2)
 #define TICK(name) \
   if (L.clock) (void)L.clock->mark(name, s)
