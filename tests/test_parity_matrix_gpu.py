@@ -45,6 +45,15 @@ MATRIX = {
     "ot_cks3d_excision_chainer": _ot_curved("cks", (16, 16, 8), (2, 2, 2), (0.6, 0.5, 0.3),
                                             (2.6, 2.5, 1.3), riemann=0, limiter=1, recovery=0,
                                             enable_heating=1),
+    # x3-independent blocks: tables of one plane, no X3 faces
+    "ot_cks2d_hll_ppm4_kastaun": _ot_curved("cks", (36, 28, 1), (2, 2, 1), (2.3, -0.5, 0.4), (3.3, 0.5, 0.9),
+                                            riemann=1, limiter=1, recovery=1, enable_heating=1),
+    "ot_cks2d_laxf_mc_chainer": _ot_curved("cks", (36, 28, 1), (1, 2, 1), (-3.3, 1.5, 0.4), (-2.3, 2.5, 0.9),
+                                           riemann=0, limiter=0, recovery=0),
+    "ot_cks2d_ppm4_kastaun_noB": _ot_curved("cks", (36, 28, 1), (2, 1, 1), (2.3, -0.5, 0.4), (3.3, 0.5, 0.9),
+                                            limiter=1, recovery=1, enable_B=0),
+    "ot_cks2d_hll_mc_onedvsq_noB": _ot_curved("cks", (36, 28, 1), (2, 2, 1), (2.3, -0.5, 0.4), (3.3, 0.5, 0.9),
+                                              riemann=1, limiter=0, recovery=2, enable_B=0),
     "ot_bl2d_hll_mc_chainer": _ot_curved("bl", (32, 32, 1), (2, 2, 1), (1.0, -0.5, 0.0),
                                          (2.0, 0.5, 1.0), riemann=1, limiter=0, recovery=0),
     "ot_mks2d_ppm4_onedvsq": _ot_curved("mks", (32, 32, 1), (1, 2, 1), (1.0, -0.5, 0.0),
