@@ -12,8 +12,10 @@
 // one ulp of x/12 and the theorem applies to every x away from underflow
 // (|x| > 2^-1018) and overflow.
 //
-// div_by: ry = 1/y comes from one IEEE division shared by all numerators of
-// a divisor.  q = RN(x ry) is within 1.5 ulp of x/y in general; the
+// div_by: ry = RN(1/y) is shared by all numerators of a divisor, from an IEEE
+// division or from quot(1, y), which is the same number (but for a divisor
+// whose significand is all ones: its reciprocal may be an ulp off, and the
+// result with it).  q = RN(x ry) is within 1.5 ulp of x/y in general; the
 // corrected result matched the IEEE quotient on every one of 6e8 random and
 // structured operand pairs (divisor significands near 1, 4/3, 3/2 and 2,
 // dense and sparse bit patterns) and is within one ulp by construction.
@@ -33,20 +35,32 @@
 // FP64 (hardware reciprocal or reciprocal square root, Newton steps, a
 // correction from the exact remainder) without the scaling and the fix-ups
 // that serve operands near the ends of the exponent range: 8 instructions
-// instead of 11, 10 instead of 18.  Where no scaling would happen the steps
+// instead of 11, 10 instead of 18.  (Newton's iteration for the reciprocal with
+// Markstein's final correction, and Goldschmidt's coupled iteration for the
+// root and half its reciprocal with two remainder corrections: Handbook of
+// Floating-Point Arithmetic, sec. 4.7 and 5.4; P. Markstein, Proc. 6th Conf.
+// Real Numbers and Computers (2004) 146-157.)  Where no scaling would happen the steps
 // are the same, so the results are: quot the IEEE quotient for x = 0 or
 // |x|, |y| and |x / y| in [2^-900, 2^900] (a divisor whose significand is all
 // ones can round a near tie the other way, with or without the scaling), root
 // the IEEE square root for x in [2^-760, 2^1000] (0 and infinity give NaN;
 // the caller excludes 0).
-// Outside, quot(x, 0) and quot(x, +-inf) give NaN, and subnormal remainders
-// can cost a unit in the last place.  The kernels use them on lapses, Lorentz
-// factors, enthalpies and wave speed sums.
+// Outside, quot(x, 0), quot(x, +-inf), a subnormal divisor and a quotient that
+// overflows give NaN, and subnormal remainders can cost a unit in the last
+// place.  The kernels use them on lapses, Lorentz factors, enthalpies and wave
+// speed sums, which leave the range only below densities of 1e-303 or where
+// squares overflow, and in the recovery's searches.  There, iterates of cells
+// without a solution pass through any value, so a division stays IEEE where
+// one that leaves the range could come back: 1Dvsq's by W^2 and W^3, 2D's
+// dP/dv^2 at v^2 = 1, its determinant and v^2.  The rest end alike: a NaN in a
+// search ends in the status that an infinity ends in.  Kastaun's
+// mu + 1e-300 divides a difference that is 0 when mu is, and eps >= 1e-300
+// enters as a term next to 1.
 // With min2 / max2 (physics_dev.h) the three sweeps of a face go from 4228 to
 // 4012 vector instructions, which are what they wait for: 3-D torus
 // 256x128x128 3.85 -> 3.82 ms per cycle, and with the Kastaun search on quot
 // and root its recovery of 128x64x64 cells 48.4 -> 45.2 us and an ensemble of
-// 24 meshes 401 -> 389 us per cycle.
+// 20 meshes 401 -> 389 us per cycle.
 //
 // The remainder is negated inside the second FMA, so a zero quotient keeps
 // the sign the IEEE division gives it (compilers that fold the negation

@@ -39,7 +39,7 @@ struct SweepSet {
 // the sweeps': 4.75 ms (a light kernel's workgroups at the sweeps' register
 // count, three wavefronts per SIMD).  Small meshes gain most: sweeps one by one ->
 // merged -> with the exchange, Orszag-Tang 256^2 97 -> 86 -> 80 us, eight
-// 32x16x16 torus blocks 169 -> 141 -> 132 us, ensemble of 24 meshes 458 -> 424 ->
+// 32x16x16 torus blocks 169 -> 141 -> 132 us, ensemble of 20 meshes 458 -> 424 ->
 // 412 us, 2-D torus 512x256 196 -> 181 -> 174 us.
 constexpr int kRun = 256;
 
