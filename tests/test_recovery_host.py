@@ -102,13 +102,18 @@ def _states(n, scale, seed, gcov, gcon):
 
 
 def _cks_point():
+    """gcov and gcon at a point where no two mirrored entries of gcov agree."""
     d = configs.orszag_tang(16, (1, 1, 1))
     d.update(metric=configs.METRIC["cks"], a=0.9375)
-    cfg, x = abi.config_from(d), np.array([0.0, 2.7, -1.9, 0.8])
-    c = np.zeros(abi.CENTRE_NCOMP)
-    dp = C.POINTER(C.c_double)
-    assert abi.lib().pangu_geometry_entry(C.byref(cfg), 0, x.ctypes.data_as(dp), c.ctypes.data_as(dp)) == abi.OK
-    return c[:16].reshape(4, 4).copy(), c[16:32].reshape(4, 4).copy()
+    cfg, dp = abi.config_from(d), C.POINTER(C.c_double)
+    rng = np.random.default_rng(1)
+    while True:
+        x = np.concatenate([[0.0], rng.uniform(-4.0, 4.0, 3)])
+        c = np.zeros(abi.CENTRE_NCOMP)
+        assert abi.lib().pangu_geometry_entry(C.byref(cfg), 0, x.ctypes.data_as(dp), c.ctypes.data_as(dp)) == abi.OK
+        g = c[:16].reshape(4, 4)
+        if g[1, 2] != g[2, 1] and g[1, 3] != g[3, 1] and g[2, 3] != g[3, 2] and np.linalg.norm(x) > 3.0:
+            return g.copy(), c[16:32].reshape(4, 4).copy()
 
 
 @pytest.mark.parametrize("scheme", [0, 1, 2, 3])
